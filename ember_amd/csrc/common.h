@@ -23,8 +23,10 @@ bool hip_ok(hipError_t err, const char *what);
 bool launch_ok(const char *kernel);
 
 // Library-owned device scratch, grown on demand and cached per device for
-// the life of the process.  Slot ids keep independent users apart.
-void *scratch(int slot, size_t bytes);
+// the life of the process.  Slot ids keep independent users apart.  optional:
+// the caller can do without, so that running out of memory gives null but
+// records no error.
+void *scratch(int slot, size_t bytes, bool optional = false);
 
 enum ScratchSlot {
     kScratchAttnDelta = 0,

@@ -7,35 +7,22 @@
 // and adds gemm_ex, which also takes either operand transposed in place
 // (a stored k x n, b stored m x k: the weight- and input-gradient products of
 // a Linear layer, ember/nn/layers.py:50-56, without materialising T(x)) and
-// the fused epilogue of linear_fwd.
-// all row-major fp32 with fp32 accumulation (v_mfma_f32_32x32x2f32; no
-// reduced-precision inputs).  The CPU path of the reference accumulates in
-// double (src/tensor/operators_cpu.c:47-60); agreement is to fp32 rounding
-// of a length-k sum, see the parity tests.
+// the fused epilogue of linear_fwd, all row-major fp32.
 //
-// Tile-aligned shapes (n % 128, m % 256, k % 16 == 0) take the fast path
-// further down (gemm_f32_dma_kernel: 128 x 256 or 256 x 256 tiles, slabs
-// copied HBM -> LDS without registers).  The general path, for any other
-// shape: a workgroup of 4 waves computes a 128 x 128 block of out, each
-// wave a 64 x 64 quadrant as 2 x 2 MFMA accumulators.  The k dimension is
-// walked in 32-wide slabs: the next slab's A (128 x 32) and B (32 x 128)
-// are loaded from HBM/L2 into registers while the current one is multiplied
-// out of LDS (two LDS buffers, one barrier per slab).  Lane half h of a wave
-// contracts k in [16h, 16h+16) of the slab, so A is read from LDS as
-// 128-bit row segments; B rows of the second half sit 32 floats further on
-// so the two lane halves read disjoint banks.  Workgroups are ordered so
-// that consecutive ones share B column panels in L2.
+// Products run on the bf16 matrix cores at fp32 precision: every operand is
+// split exactly into three bf16 parts (split_bf16.h), and six of the nine
+// part products are accumulated in fp32.  One kernel covers every shape,
+// orientation and alignment; choose_shape picks its tile.
+#include <math.h>
+
+#include <type_traits>
+
 #include "common.h"
-#include "lds_dma.h"
 #include "mfma.h"
+#include "split_bf16.h"
 
 namespace ember {
 namespace {
-
-constexpr int kThreads = 256;
-constexpr int BM = 128, BN = 128, BK = 32;
-constexpr int ASTR = BK + 4;  // padded A row in LDS
-constexpr int BBUF = BK * BN + 32;
 
 struct GemmArgs {
     const float *a, *b;
@@ -45,7 +32,7 @@ struct GemmArgs {
     int ta, tb;          // a stored k x n / b stored m x k
     int64_t sa, sb, sc;  // batch strides (elements)
     int tiles_n, tiles_m;
-    int kchunk;          // split-K: k range of one blockIdx.z (multiple of 16)
+    int kchunk;          // split-K: k range of one blockIdx.z (multiple of 32)
     float *part;         // split-K partial sums [ksplit][batch][n][m]
     // Epilogue (all optional): out = act(acc + bias[col]) + residual, with
     // pre = acc + bias stored before the activation; residual and pre use
@@ -73,225 +60,180 @@ __device__ __forceinline__ float epilogue(const GemmArgs &g, float v, int64_t of
     return v;
 }
 
-__device__ __forceinline__ int bs_index(int kr, int col)
+__device__ __forceinline__ bool is_tiny(float m)
 {
-    return kr * BN + (kr >= BK / 2 ? 32 : 0) + col;
+    return m > 0.0f && m < kSplitTiny;
 }
 
-// Loads one slab into registers: A rows row0.., cols k0..k0+31; B rows k0..,
-// cols col0..col0+127.  Out-of-range elements read as 0.
-template <bool VEC>
-__device__ __forceinline__ void load_slab(const GemmArgs &g, const float *A, const float *B, int row0,
-                                          int col0, int k0, int tid, f32x4 (&ra)[4], f32x4 (&rb)[4])
-{
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int idx = it * kThreads + tid;  // 0..1023
-        {   // A: 128 rows x 8 float4
-            const int r = idx >> 3, c4 = idx & 7;
-            const int row = row0 + r, col = k0 + 4 * c4;
-            f32x4 v = {0.f, 0.f, 0.f, 0.f};
-            if (VEC && !g.ta) {
-                if (row < g.n && col < g.k) v = *(const f32x4 *)(A + (int64_t)row * g.lda + col);
-            } else if (row < g.n) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (col + j < g.k)
-                        v[j] = g.ta ? A[(int64_t)(col + j) * g.lda + row]
-                                    : A[(int64_t)row * g.lda + col + j];
-            }
-            ra[it] = v;
-        }
-        {   // B: 32 rows x 32 float4
-            const int r = idx >> 5, c4 = idx & 31;
-            const int row = k0 + r, col = col0 + 4 * c4;
-            f32x4 v = {0.f, 0.f, 0.f, 0.f};
-            if (VEC && !g.tb) {
-                if (row < g.k && col < g.m) v = *(const f32x4 *)(B + (int64_t)row * g.ldb + col);
-            } else if (row < g.k) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (col + j < g.m)
-                        v[j] = g.tb ? B[(int64_t)(col + j) * g.ldb + row]
-                                    : B[(int64_t)row * g.ldb + col + j];
-            }
-            rb[it] = v;
-        }
+// One operand's share of a k-slab: R tile rows (rows of a, columns of b) by
+// BK of k, loaded into registers by NT threads, split, and stored to LDS as
+// three bf16 planes.  A thread holds G groups of 8 consecutive k of one row.
+// KC: the operand is stored with k contiguous (a n x k, b m x k): a group is
+// two 16-byte loads, and BK/8 neighbouring lanes share a row.  Otherwise (a
+// k x n, b k x m) lanes run along the rows and a group is 8 dword loads, each
+// 256 contiguous bytes per wave.  Either way a group's 8 elements are k
+// neighbours, so its parts are stored as one 16-byte LDS write per plane.
+// LDS: row r's 16-byte unit q of a plane sits at unit r * BK/8 + (q ^ swz(r)),
+// with swz chosen so that 16 neighbouring rows of one q, which a quarter wave
+// reads or writes together, fall on different banks.
+template <int R, int BK, int NT, bool KC>
+struct Operand {
+    static constexpr int Q = BK / 8;             // 16-byte units per row and plane
+    static constexpr int G = R * Q / NT;         // groups per thread
+    static constexpr int kPlane = R * Q;         // units per plane
+    static_assert(G >= 1 && G * NT == R * Q, "whole groups per thread");
+    static_assert(Q == 2 || Q == 4, "swizzle below");
+    static_assert(KC || R % 64 == 0, "a wave's lanes stay in one k row");
+
+    const float *p[G];  // KC: this lane's group at the slab to load; else the wave's k row
+    unsigned voff;      // !KC: this lane's byte offset from there
+    int kq[G];          // the group's k offset within the slab
+    float v[G][8];
+    float big[G];       // largest magnitude the group's row has shown
+    unsigned neg[G];    // sign_of the group's row
+    unsigned s[G][3][2];  // two split pairs: hi, mid, lo
+
+    static __device__ __forceinline__ int unit(int r, int q)
+    {
+        return r * Q + (q ^ (Q == 2 ? (r >> 3) & 1 : (r >> 2) & 3));
     }
-}
-
-__device__ __forceinline__ void store_slab(float *As, float *Bs, int tid, const f32x4 (&ra)[4],
-                                           const f32x4 (&rb)[4])
-{
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int idx = it * kThreads + tid;
-        {
-            const int r = idx >> 3, c4 = idx & 7;
-            *(f32x4 *)&As[r * ASTR + 4 * c4] = ra[it];
-        }
-        {
-            const int r = idx >> 5, c4 = idx & 31;
-            *(f32x4 *)&Bs[bs_index(r, 4 * c4)] = rb[it];
-        }
+    static __device__ __forceinline__ int row_of(int tid, int g)
+    {
+        const int i = tid + NT * g;
+        return KC ? i / Q : i % R;
     }
-}
-
-template <bool VEC>
-__global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(GemmArgs g)
-{
-    __shared__ float As[2][BM * ASTR];
-    __shared__ float Bs[2][BBUF];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int w = tid >> 6;
-    const int h32 = lane >> 5;
-    const int l32 = lane & 31;
-    const int wr = w >> 1, wc = w & 1;
-
-    // Column panels vary slowest within a group of 8 row tiles so that
-    // neighbouring workgroups reuse the same B panel from L2.
-    const int tile = blockIdx.x;
-    constexpr int GROUP = 8;
-    const int per_group = GROUP * g.tiles_m;
-    const int grp = tile / per_group;
-    const int first_row_tile = grp * GROUP;
-    const int rows_in_grp = min(GROUP, g.tiles_n - first_row_tile);
-    const int in_grp = tile - grp * per_group;
-    const int tn = first_row_tile + in_grp % rows_in_grp;
-    const int tm = in_grp / rows_in_grp;
-
-    const int row0 = tn * BM;
-    const int col0 = tm * BN;
-    const float *A = g.a + (int64_t)blockIdx.y * g.sa;
-    const float *B = g.b + (int64_t)blockIdx.y * g.sb;
-    float *C = g.c + (int64_t)blockIdx.y * g.sc;
-
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
-
-    f32x4 ra[4], rb[4];
-    const int nslab = (g.k + BK - 1) / BK;
-    load_slab<VEC>(g, A, B, row0, col0, 0, tid, ra, rb);
-    store_slab(As[0], Bs[0], tid, ra, rb);
-    __syncthreads();
-
-    for (int s = 0; s < nslab; ++s) {
-        const int cur = s & 1;
-        if (s + 1 < nslab) load_slab<VEC>(g, A, B, row0, col0, (s + 1) * BK, tid, ra, rb);
-        const float *as = As[cur];
-        const float *bs = Bs[cur];
-#pragma unroll
-        for (int kk = 0; kk < BK / 2; kk += 4) {
-            f32x4 af[2];
-#pragma unroll
-            for (int rb2 = 0; rb2 < 2; ++rb2)
-                af[rb2] = *(const f32x4 *)&as[(64 * wr + 32 * rb2 + l32) * ASTR + h32 * (BK / 2) + kk];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int kr = h32 * (BK / 2) + kk + j;
-                float bf[2];
-#pragma unroll
-                for (int cb = 0; cb < 2; ++cb) bf[cb] = bs[bs_index(kr, 64 * wc + 32 * cb + l32)];
-#pragma unroll
-                for (int rb2 = 0; rb2 < 2; ++rb2)
-#pragma unroll
-                    for (int cb = 0; cb < 2; ++cb)
-                        acc[rb2][cb] = mfma_32x32x2(af[rb2][j], bf[cb], acc[rb2][cb]);
-            }
-        }
-        if (s + 1 < nslab) store_slab(As[cur ^ 1], Bs[cur ^ 1], tid, ra, rb);
-        __syncthreads();
+    static __device__ __forceinline__ int unit_of(int tid, int g)
+    {
+        const int i = tid + NT * g;
+        return KC ? i % Q : i / R;
     }
 
+    // base: the matrix; rows past `rows` re-read the last one (their results
+    // are not stored).
+    __device__ __forceinline__ void init(const float *base, int64_t ld, int row0, int rows, int kbeg, int tid)
+    {
 #pragma unroll
-    for (int rb2 = 0; rb2 < 2; ++rb2) {
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-            const int col = col0 + 64 * wc + 32 * cb + l32;
-            if (col >= g.m) continue;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = row0 + 64 * wr + 32 * rb2 + acc_row(i, h32);
-                if (row < g.n) {
-                    const int64_t off = (int64_t)blockIdx.y * g.sc + (int64_t)row * g.m + col;
-                    C[(int64_t)row * g.m + col] = epilogue(g, acc[rb2][cb][i], off, col);
-                }
-            }
+        for (int g = 0; g < G; ++g) {
+            const int r = min(row_of(tid, g), rows - 1 - row0);
+            int q = unit_of(tid, g);
+            if (!KC) q = __builtin_amdgcn_readfirstlane(q);  // one k row per wave: scalar addresses
+            kq[g] = 8 * q;
+            neg[g] = sign_of(row0 + row_of(tid, g));
+            p[g] = KC ? base + (int64_t)(row0 + r) * ld + kbeg + 8 * q : base + (int64_t)(kbeg + 8 * q) * ld + row0;
+            if (!KC) voff = 4u * (unsigned)r;
+            big[g] = 0.0f;
         }
     }
-}
+    __device__ __forceinline__ float at(int g, int j, int64_t ld) const
+    {
+        if (KC) return p[g][j];
+        return *(const float *)((const char *)(p[g] + j * ld) + voff);
+    }
+    // Loads group g of a whole slab.
+    __device__ __forceinline__ void load_group(int64_t ld, int g)
+    {
+        typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+        if (KC) {
+            const f32x4u x = *(const f32x4u *)p[g], y = *(const f32x4u *)(p[g] + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[g][j] = x[j], v[g][4 + j] = y[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[g][j] = at(g, j, ld);
+        }
+    }
+    __device__ __forceinline__ void load(int64_t ld)
+    {
+#pragma unroll
+        for (int g = 0; g < G; ++g) load_group(ld, g);
+    }
+    // Loads a partial slab of `len` k.
+    __device__ __forceinline__ void load_part(int64_t ld, int len)
+    {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[g][j] = kq[g] + j < len ? at(g, j, ld) : 0.0f;
+    }
+    // Moves on by k.
+    __device__ __forceinline__ void advance(int64_t ld, int k)
+    {
+#pragma unroll
+        for (int g = 0; g < G; ++g) p[g] += KC ? (int64_t)k : k * ld;
+    }
+    // Splits pair i (of 4) of group g; after every second one half a unit of
+    // each plane is stored.
+    __device__ __forceinline__ void split_store(int g, int i, u32x4 *__restrict__ lds, int tid)
+    {
+        const float x = flip(v[g][2 * i], neg[g]), y = flip(v[g][2 * i + 1], neg[g]);
+        big[g] = fmaxf(big[g], fmaxf(fabsf(x), fabsf(y)));
+        split_pair(x, y, s[g][0][i & 1], s[g][1][i & 1], s[g][2][i & 1]);
+        if (i & 1) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            u32x2 *const to = (u32x2 *)lds + 2 * unit(row_of(tid, g), unit_of(tid, g)) + i / 2;
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) to[2 * pl * kPlane] = u32x2{s[g][pl][0], s[g][pl][1]};
+        }
+    }
+    __device__ __forceinline__ void store(u32x4 *__restrict__ lds, int tid)
+    {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) split_store(g, i, lds, tid);
+    }
+    __device__ __forceinline__ bool tiny() const
+    {
+        bool t = false;
+#pragma unroll
+        for (int g = 0; g < G; ++g) t |= is_tiny(big[g]);
+        return t;
+    }
+    __device__ __forceinline__ void row_max(unsigned *m, int tid) const
+    {
+#pragma unroll
+        for (int g = 0; g < G; ++g) atomicMax(&m[row_of(tid, g)], __builtin_bit_cast(unsigned, big[g]));
+    }
+};
 
-// ---------------------------------------------------------------------------
-// Fast path for tile-aligned shapes (n % 128 == 0, m % 256 == 0, k % 16 == 0,
-// 16-byte aligned operands): 128 x 256 block of out per workgroup, 64 x 128
-// per wave as 2 x 4 accumulators, two workgroups per CU.
-//   * k is walked in slabs of 16, copied HBM -> LDS directly
-//     (buffer_load_dwordx4 ... lds, no registers) one slab ahead into the
-//     other of two buffers; one barrier per slab.
-//   * A slab, a stored n x k: 128 tile rows padded to 20 floats, so the A
-//     operand (one row per lane, 4 k per ds_read_b128) hits 16 different
-//     bank groups.  a stored k x n (TA): 16 k-rows of 128 floats; a lane
-//     reads two neighbouring tile rows with one ds_read_b64 and uses them as
-//     the two row blocks of its wave, i.e. MFMA row r of row block rb is tile
-//     row 2r + rb of the wave's 64 (undone in the store).
-//   * B slab, b stored k x m: 16 rows of 256, a lane reads 4 consecutive
-//     columns with one ds_read_b128, one per accumulator column block
-//     (column = 4*lane + cb).  b stored m x k (TB): 256 columns padded to 20
-//     floats, a lane reads 4 k of its column with one ds_read_b128 (column =
-//     32*cb + lane).  Either way each B read feeds 8 MFMAs.
-//   * every LDS address in the loop is a per-lane base plus a compile-time
-//     offset.
+// A TM x TN block of out per workgroup of WR x WC waves, each 32*RB x 32*CB.
+// What bounds it: the matrix cores, and at 4096^3 the power limit with them
+// (72 % of cycles busy, at 1.70 GHz; the same launch on constant operands
+// holds 2.28 GHz): 933 -> 601 us, 147 -> 228 TFLOP/s against the fp32
+// instruction's kernel this replaced.  Splitting costs 5.5 vector operations
+// per element staged (2.2 per matrix instruction in the 256 x 256 tile, 4 are
+// free beside one), so operands are split once, when they enter LDS, and not
+// by each wave that reads them.
+//   * k is walked in slabs of BK through two LDS buffers, one barrier per
+//     slab: while slab s is multiplied, slab s+1 (in registers) is split and
+//     stored to the other buffer and slab s+2 is requested.
 //   * tiles are numbered so that the tiles one XCD runs (workgroup ids are
-//     dealt to the 8 XCDs round-robin) are contiguous, and within that
-//     range grouped 8 row tiles per B column panel for L2 reuse.
-//   * split-K (SPLIT): blockIdx.z walks k in [z*kchunk, (z+1)*kchunk) and
+//     dealt to the 8 XCDs round-robin) are contiguous, and within that range
+//     grouped 8 row tiles per b column panel for L2 reuse.
+//   * split-K (g.part): blockIdx.z walks k in [z*kchunk, (z+1)*kchunk) and
 //     stores its raw sums to part; gemm_splitk_reduce adds the splits in
 //     order and applies the epilogue, so results do not depend on timing.
-constexpr int FM = 128, FN = 256, FK = 16;
-constexpr int FASTR = FK + 4;  // padded row of a k-contiguous slab
-
-template <bool TA, int TM = FM> struct ASlab {
-    static_assert(!TA || TM == 128, "a stored k x n: one 1 KiB copy is two 128-float rows");
-    static constexpr int kBuf = TA ? FK * TM : TM * FASTR;     // floats
-    static constexpr int kCopies = kBuf / 256;                  // 1 KiB copies
-};
-template <bool TB> struct BSlab {
-    static constexpr int kBuf = TB ? FN * FASTR : FK * FN;
-    static constexpr int kCopies = kBuf / 256;                  // 20 / 16
-};
-
-// TM = 128 (4 waves, 2 workgroups per CU) or 256 (8 waves, 1 per CU: the
-// same 64 x 128 per wave, a third less L2 -> LDS traffic per flop).
-// KG = 2 (TM = 128 only): two groups of 4 waves per workgroup, one per CU,
-// each group with its own LDS buffers and the whole 128 x 256 tile; group 0
-// multiplies the even k-slabs, group 1 the odd ones, and group 1's sums are
-// added to group 0's through LDS before the store.  For outputs with no more
-// tiles than CUs: two waves per SIMD instead of one, no extra HBM traffic.
-template <bool TA, bool TB, bool SPLIT, int TM = FM, int KG = 1>
-__global__ __launch_bounds__(TM * 2 * KG, TM == 128 && KG == 1 ? 2 : 1) void gemm_f32_dma_kernel(GemmArgs g)
+//   * a wave whose sums are not finite, or whose workgroup met a row too
+//     small to split (split_bf16.h), computes its block again from global
+//     memory with the fp32 instruction.
+template <int TM, int TN, int WR, int WC, int BK, int PER_CU, bool TWO, bool TA, bool TB>
+__global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmArgs g)
 {
-    static_assert(KG == 1 || (KG == 2 && TM == 128 && !SPLIT), "k groups: 128-row tiles, no split-K");
-    constexpr int NW = TM / 32;  // waves per group: TM/64 rows x 2 columns of 64 x 128
-    constexpr int ABUF = ASlab<TA, TM>::kBuf, BBUF_ = BSlab<TB>::kBuf;
-    constexpr int ACOP = ASlab<TA, TM>::kCopies, BCOP = BSlab<TB>::kCopies;
-    __shared__ float As0[KG * ABUF], As1[KG * ABUF];
-    __shared__ float Bs0[KG * BBUF_], Bs1[KG * BBUF_];
+    constexpr int NT = 64 * WR * WC;
+    constexpr int RB = TM / WR / 32, CB = TN / WC / 32;
+    typedef Operand<TM, BK, NT, !TA> OA;
+    typedef Operand<TN, BK, NT, TB> OB;
+    
+    __shared__ u32x4 As0[3 * OA::kPlane], As1[3 * OA::kPlane];
+    __shared__ u32x4 Bs0[3 * OB::kPlane], Bs1[3 * OB::kPlane];
+    __shared__ int tiny_row;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    // Wave index made provably uniform: the per-wave copy counts and LDS
-    // destinations below then use scalar branches and registers.
-    const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grpk = KG == 1 ? 0 : wg / NW;  // k group
-    const int w = KG == 1 ? wg : wg - grpk * NW;  // wave within the group
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h32 = lane >> 5;
     const int l32 = lane & 31;
-    const int wr = w >> 1, wc = w & 1;
+    const int wr = w / WC, wc = w % WC;
 
     const int ntiles = g.tiles_n * g.tiles_m;
     int tile = blockIdx.x;
@@ -302,244 +244,272 @@ __global__ __launch_bounds__(TM * 2 * KG, TM == 128 && KG == 1 ? 2 : 1) void gem
     const int first = grp * GROUP;
     const int rows_in_grp = min(GROUP, g.tiles_n - first);
     const int in_grp = tile - grp * per_group;
-    // The tile origin is computed with vector integer division; made
-    // provably uniform here, it stays in scalar registers and the buffer
-    // descriptors built from it need no per-lane (waterfall) handling.
+    // Provably uniform, so that the operand addresses keep scalar parts.
     const int row0 = __builtin_amdgcn_readfirstlane((first + in_grp % rows_in_grp) * TM);
-    const int col0 = __builtin_amdgcn_readfirstlane((in_grp / rows_in_grp) * FN);
+    const int col0 = __builtin_amdgcn_readfirstlane((in_grp / rows_in_grp) * TN);
 
     int kbeg = 0, kend = g.k;
-    if (SPLIT) {
+    if (g.part) {
         kbeg = blockIdx.z * g.kchunk;
         kend = min(g.k, kbeg + g.kchunk);
     }
-    // Tile origins; slab k0 (absolute) is added per fetch.
-    const float *A = g.a + (int64_t)blockIdx.y * g.sa + (TA ? (int64_t)row0 : (int64_t)row0 * g.lda);
-    const float *B = g.b + (int64_t)blockIdx.y * g.sb + (TB ? (int64_t)col0 * g.ldb : (int64_t)col0);
+    const float *A = g.a + (int64_t)blockIdx.y * g.sa;
+    const float *B = g.b + (int64_t)blockIdx.y * g.sb;
 
-    // Per-lane byte offsets of the 1 KiB copies this wave issues (copy
-    // t = w + NW*s), below 2^32 because lda, ldb < 2^22 (checked on the host).
-    constexpr int AS = (ACOP + NW - 1) / NW, BS = (BCOP + NW - 1) / NW;
-    unsigned aoff[AS], boff[BS];
+    // TWO: the five small products of a pair of operands are summed apart
+    // from the large one, so that each sum is rounded less often.
+    f32x16 acc[RB][CB], low[TWO ? RB : 1][TWO ? CB : 1];
 #pragma unroll
-    for (int s = 0; s < AS; ++s) {
-        const int t = w + NW * s;
-        if (TA) {  // copy t: k-rows 2t, 2t+1, 32 chunks each
-            aoff[s] = 4u * (unsigned)((2 * t + h32) * g.lda + 4 * l32);
-        } else {   // row p / 5, chunk p % 5 (chunk 4 is row padding: re-read chunk 0)
-            const int p = 64 * t + lane;
-            const int r = p / (FASTR / 4), c = p - r * (FASTR / 4);
-            aoff[s] = 4u * (unsigned)(r * g.lda + 4 * (c < 4 ? c : 0));
-        }
-    }
+    for (int i = 0; i < RB; ++i)
 #pragma unroll
-    for (int s = 0; s < BS; ++s) {
-        const int t = w + NW * s;
-        if (TB) {
-            const int p = 64 * t + lane;
-            const int r = p / (FASTR / 4), c = p - r * (FASTR / 4);
-            boff[s] = 4u * (unsigned)(r * g.ldb + 4 * (c < 4 ? c : 0));
-        } else {   // copy t: k-row t
-            boff[s] = 4u * (unsigned)(t * g.ldb + 4 * lane);
+        for (int j = 0; j < CB; ++j) {
+            acc[i][j] = zero16();
+            if (TWO) low[i][j] = zero16();
         }
-    }
 
-    auto fetch = [&](int k0, float *__restrict__ as, float *__restrict__ bs) {
-        const __amdgpu_buffer_rsrc_t ra = dma_rsrc(TA ? A + (int64_t)k0 * g.lda : A + k0);
+    OA oa;
+    OB ob;
+    // Slab 0 takes what k leaves over, the others are whole, so that the loop
+    // has no bounds on k and the short slab's guarded loads share the
+    // prologue's wait.
+    const int nslab = (kend - kbeg + BK - 1) / BK;
+    const int first_k = kend - kbeg - (nslab - 1) * BK;
+    const int arow = 32 * RB * wr + l32, bcol = 32 * CB * wc + l32;
+    // Multiplies slab s (in as, bs) while slab s + 1 (in registers) is split
+    // and stored to the other buffer and slab s + 2 is loaded.  Past the last
+    // slab the last one is loaded again and not used: no branches here.
+    // The products are cut into chunks of one b block; each chunk reads the
+    // operands of the next one, the last, behind the barrier, those of the
+    // next slab, and the chunks before it take an even share of the splitting.
+    constexpr int KS = BK / 16, NC = KS * CB;
+    static_assert(NC % 2 == 0, "b operands alternate between two register sets");
+    constexpr int NU = 4 * (OA::G + OB::G);  // pairs to split
+    constexpr int NS = (NC - 1) * RB * 6;    // products they are spread over
+    Split8 af[2][RB], bf[2];
+    auto read_a = [&](const u32x4 *__restrict__ as, int ks, Split8 (&f)[RB]) {
 #pragma unroll
-        for (int s = 0; s < AS; ++s)
-            if (w + NW * s < ACOP) dma16_buf(ra, aoff[s], as + 256 * (w + NW * s));
-        const __amdgpu_buffer_rsrc_t rb = dma_rsrc(TB ? B + k0 : B + (int64_t)k0 * g.ldb);
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int s = 0; s < BS; ++s)
-            if (w + NW * s < BCOP) dma16_buf(rb, boff[s], bs + 256 * (w + NW * s));
+            for (int pl = 0; pl < 3; ++pl)
+                f[rb].part[pl] = as[pl * OA::kPlane + 32 * rb * OA::Q + OA::unit(arow, 2 * ks + h32)];
     };
-
-    f32x16 acc[2][4];
+    auto read_b = [&](const u32x4 *__restrict__ bs, int ks, int cb, Split8 &f) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int pl = 0; pl < 3; ++pl)
+            f.part[pl] = bs[pl * OB::kPlane + 32 * cb * OB::Q + OB::unit(bcol, 2 * ks + h32)];
+    };
+    auto step = [&](auto parity, auto only, int s, const u32x4 *__restrict__ as, const u32x4 *__restrict__ bs,
+                    u32x4 *__restrict__ an, u32x4 *__restrict__ bn) {
+        constexpr int PA = decltype(parity)::value;
+        constexpr bool ONLY = decltype(only)::value;  // the one slab: nothing to stage
+        const int k = s + 3 < nslab ? BK : 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = zero16();
-
-    const int abase = TA ? 8 * h32 * TM + 64 * wr + 2 * l32 : (64 * wr + l32) * FASTR + 8 * h32;
-    const int bbase = TB ? (128 * wc + l32) * FASTR + 8 * h32 : 8 * h32 * FN + 128 * wc + 4 * l32;
-    auto slab = [&](const float *__restrict__ as, const float *__restrict__ bs) {
-#pragma unroll
-        for (int kk = 0; kk < 8; kk += 4) {
-            f32x4 af[2];
-            if (TA) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const f32x2 v = *(const f32x2 *)&as[abase + (kk + j) * TM];
-                    af[0][j] = v[0];
-                    af[1][j] = v[1];
-                }
-            } else {
-#pragma unroll
-                for (int rb = 0; rb < 2; ++rb) af[rb] = *(const f32x4 *)&as[abase + rb * 32 * FASTR + kk];
+        for (int c = 0; c < NC; ++c) {
+            const int ks = c / CB, cb = c % CB;
+            if (c + 1 < NC) {
+                if ((c + 1) % CB == 0) read_a(as, (c + 1) / CB, af[(PA + (c + 1) / CB) & 1]);
+                read_b(bs, (c + 1) / CB, (c + 1) % CB, bf[(c + 1) & 1]);
+            } else if (!ONLY) {
+                __syncthreads();
+                read_a(an, 0, af[(PA + KS) & 1]);
+                read_b(bn, 0, 0, bf[0]);
             }
-            f32x4 bt[4];
-            if (TB) {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb) bt[cb] = *(const f32x4 *)&bs[bbase + cb * 32 * FASTR + kk];
-            }
-            if (TB) {
-                // Column block outermost: the MFMAs of block cb need only its
-                // own B read, so the later reads overlap earlier products
-                // (k-step innermost would need all four reads before the
-                // first MFMA: 12 % slower with one workgroup per CU).  Each
-                // accumulator still adds its k-steps in the same order.
+            for (int t = 0; t < 6; ++t) {
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb)
+                for (int rb = 0; rb < RB; ++rb) {
+                    const Split8 &x = af[(PA + ks) & 1][rb], &y = bf[c & 1];
+                    if constexpr (TWO)
+                        mfma_split_term(t, x, y, t == 5 ? acc[rb][cb] : low[rb][cb]);
+                    else
+                        mfma_split_term(t, x, y, acc[rb][cb]);
+                    const int done = (c * 6 + t) * RB + rb;
 #pragma unroll
-                    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[rb][cb] = mfma_32x32x2(af[rb][j], bt[cb][j], acc[rb][cb]);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const f32x4 bf = *(const f32x4 *)&bs[bbase + (kk + j) * FN];
-#pragma unroll
-                    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-                        for (int cb = 0; cb < 4; ++cb) acc[rb][cb] = mfma_32x32x2(af[rb][j], bf[cb], acc[rb][cb]);
+                    for (int u = 0; u < NU; ++u) {
+                        if (ONLY || done >= NS || u * NS / NU != done) continue;
+                        if (u < 4 * OA::G) {
+                            oa.split_store(u / 4, u % 4, an, tid);
+                            if (u % 4 == 3) oa.load_group(g.lda, u / 4);
+                        } else {
+                            ob.split_store(u / 4 - OA::G, u % 4, bn, tid);
+                            if (u % 4 == 3) ob.load_group(g.ldb, u / 4 - OA::G);
+                        }
+                    }
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        oa.advance(g.lda, k);
+        ob.advance(g.ldb, k);
     };
 
-    // This group's buffers and slabs: slab j of the group is slab
-    // KG*j + grpk of the tile (the host launches KG = 2 only when the slab
-    // count is even, so both groups meet the same barriers).
-    float *const as0 = As0 + grpk * ABUF, *const as1 = As1 + grpk * ABUF;
-    float *const bs0 = Bs0 + grpk * BBUF_, *const bs1 = Bs1 + grpk * BBUF_;
-    const int nslab = (kend - kbeg) / FK / KG;
-    auto kslab = [&](int j) { return kbeg + (KG * j + grpk) * FK; };
+    if (tid == 0) tiny_row = 0;
     if (nslab > 0) {
-        fetch(kslab(0), as0, bs0);
-        wait_vmem();
-        __syncthreads();
-    }
-    // Two slabs per trip so that each buffer is a distinct LDS object: the
-    // compiler then knows the copy into one does not feed reads of the other.
-    for (int s = 0; s < nslab; s += 2) {
-        if (s + 1 < nslab) fetch(kslab(s + 1), as1, bs1);
-        slab(as0, bs0);
-        wait_vmem();
-        __syncthreads();
-        if (s + 1 < nslab) {
-            if (s + 2 < nslab) fetch(kslab(s + 2), as0, bs0);
-            slab(as1, bs1);
-            wait_vmem();
-            __syncthreads();
+        oa.init(A, g.lda, row0, g.n, kbeg, tid);
+        ob.init(B, g.ldb, col0, g.m, kbeg, tid);
+        if (first_k == BK) {
+            oa.load(g.lda);
+            ob.load(g.ldb);
+        } else {
+            oa.load_part(g.lda, first_k);
+            ob.load_part(g.ldb, first_k);
         }
-    }
-    if constexpr (KG == 2) {
-        // Group 1's sums to group 0, one row block at a time through the B
-        // buffers (free after the loop's last barrier): wave w of group 1
-        // writes acc[rb][0..3] lane-linearly (4096 floats) at xb, the wave
-        // of group 0 with the same w reads them back.  Sums in a fixed order
-        // (even slabs + odd slabs).
-        static_assert(2 * BBUF_ >= 2 * 4096, "exchange area: two waves per B buffer");
-        float *const xb = (w < 2 ? Bs0 : Bs1) + (w & 1) * 4096 + 4 * lane;
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-            if (grpk == 1) {
-#pragma unroll
-                for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        *(f32x4 *)&xb[(cb * 4 + q) * 256] =
-                            f32x4{acc[rb][cb][4 * q], acc[rb][cb][4 * q + 1], acc[rb][cb][4 * q + 2], acc[rb][cb][4 * q + 3]};
-            }
-            __syncthreads();
-            if (grpk == 0) {
-#pragma unroll
-                for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const f32x4 o = *(const f32x4 *)&xb[(cb * 4 + q) * 256];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[rb][cb][4 * q + e] += o[e];
-                    }
-            }
-            __syncthreads();
+        if (nslab > 1) {
+            oa.advance(g.lda, first_k);
+            ob.advance(g.ldb, first_k);
         }
-        if (grpk == 1) return;
+        oa.store(As0, tid);
+        ob.store(Bs0, tid);
+        if (nslab > 1) {
+            oa.load(g.lda);
+            ob.load(g.ldb);
+            oa.advance(g.lda, nslab > 2 ? BK : 0);
+            ob.advance(g.ldb, nslab > 2 ? BK : 0);
+        }
+        __syncthreads();
+        read_a(As0, 0, af[0]);
+        read_b(Bs0, 0, 0, bf[0]);
+        // Two slabs per trip so that each buffer is a distinct LDS object:
+        // the compiler then knows a store to one does not feed reads of the
+        // other.
+        typedef std::integral_constant<int, 0> zero;
+        if (nslab == 1) step(zero{}, std::true_type{}, 0, As0, Bs0, As1, Bs1);
+        for (int s = 0; nslab > 1;) {
+            step(zero{}, std::false_type{}, s, As0, Bs0, As1, Bs1);
+            if (++s == nslab) break;
+            step(std::integral_constant<int, KS & 1>{}, std::false_type{}, s, As1, Bs1, As0, Bs0);
+            if (++s == nslab) break;
+        }
+        __syncthreads();  // the operands read ahead, before the buffers are used again below
+    }
+    if (TWO) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) acc[i][j] += low[i][j];
     }
 
-    // Output: row(rb, i) and col(cb) as the operand layouts above define them.
-    const int64_t zoff = SPLIT ? ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * g.sc
-                               : (int64_t)blockIdx.y * g.sc;
-    const int64_t tile_off = zoff + (int64_t)row0 * g.m + col0;
-    float *C = (SPLIT ? g.part : g.c) + tile_off;
-    const bool epi = !SPLIT && (g.bias || g.pre || g.act || g.residual);
-    // This lane's output columns (within the tile) for accumulator column
-    // block cb: 4*l32 + cb (+128*wc) in the normal layout, 32*cb + l32 with
-    // b transposed.  The epilogue's bias is loaded once per column.
-    auto colof = [&](int cb) { return 128 * wc + (TB ? 32 * cb + l32 : 4 * l32 + cb); };
-    f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-    if (epi && g.bias) {
+    // Anything the split cannot carry (see split_bf16.h): do this wave's
+    // block again with the fp32 instruction.
+    if (nslab > 0) {
+        if (oa.tiny() || ob.tiny()) tiny_row = 1;
+        __syncthreads();
+        if (tiny_row) {
+            // A thread saw only its share of a row's k: take the row's maximum.
+            unsigned *const ma = (unsigned *)As0, *const mb = (unsigned *)Bs0;
+            for (int i = tid; i < TM; i += NT) ma[i] = 0;
+            for (int i = tid; i < TN; i += NT) mb[i] = 0;
+            __syncthreads();
+            oa.row_max(ma, tid);
+            ob.row_max(mb, tid);
+            if (tid == 0) tiny_row = 0;
+            __syncthreads();
+            bool tiny = false;
+            for (int i = tid; i < TM; i += NT) tiny |= is_tiny(__builtin_bit_cast(float, ma[i]));
+            for (int i = tid; i < TN; i += NT) tiny |= is_tiny(__builtin_bit_cast(float, mb[i]));
+            if (tiny) tiny_row = 1;
+            __syncthreads();
+        }
+        float probe = 0.0f;
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) bv[cb] = g.bias[col0 + colof(cb)];
-    }
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+            for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = TA ? 64 * wr + 2 * acc_row(i, h32) + rb : 64 * wr + 32 * rb + acc_row(i, h32);
-            f32x4 v;
+                for (int i = 0; i < 16; ++i) probe = fmaf(acc[rb][cb][i], 0.0f, probe);
+        if (__ballot(probe != 0.0f) != 0 || tiny_row) {
+            const float *ap[RB], *bp[CB];
+            unsigned aneg[RB], bneg[CB];
 #pragma unroll
-            for (int cb = 0; cb < 4; ++cb) v[cb] = acc[rb][cb][i];
-            const int64_t roff = (int64_t)row * g.m;
-            if (epi) {
-                // out = act(acc + bias) + residual, pre = acc + bias.
-#pragma clang fp contract(off)
-                if (g.bias) v += bv;
-                if (TB) {
-#pragma unroll
-                    for (int cb = 0; cb < 4; ++cb) {
-                        if (g.pre) g.pre[tile_off + roff + colof(cb)] = v[cb];
-                        if (g.act == 1) v[cb] = gelu08(v[cb]);
-                        if (g.residual) v[cb] += g.residual[tile_off + roff + colof(cb)];
-                    }
-                } else {
-                    if (g.pre) *(f32x4 *)&g.pre[tile_off + roff + colof(0)] = v;
-                    if (g.act == 1) {
-#pragma unroll
-                        for (int cb = 0; cb < 4; ++cb) v[cb] = gelu08(v[cb]);
-                    }
-                    if (g.residual) v += *(const f32x4 *)&g.residual[tile_off + roff + colof(0)];
-                }
+            for (int rb = 0; rb < RB; ++rb) {
+                const int64_t r = min(row0 + arow + 32 * rb, g.n - 1);
+                ap[rb] = A + (TA ? r : r * g.lda);
+                aneg[rb] = sign_of(row0 + arow + 32 * rb);
             }
-            if (TB) {
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb) C[roff + colof(cb)] = v[cb];
-            } else {
-                *(f32x4 *)&C[roff + colof(0)] = v;
+            for (int cb = 0; cb < CB; ++cb) {
+                const int64_t c = min(col0 + bcol + 32 * cb, g.m - 1);
+                bp[cb] = B + (TB ? c * g.ldb : c);
+                bneg[cb] = sign_of(col0 + bcol + 32 * cb);
+            }
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = zero16();
+            for (int k0 = kbeg; k0 < kend; k0 += 2) {
+                const int64_t k = k0 + h32;
+                float av[RB], bv[CB];
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    av[rb] = flip(k < kend ? ap[rb][TA ? k * g.lda : k] : 0.0f, aneg[rb]);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+                    bv[cb] = flip(k < kend ? bp[cb][TB ? k : k * g.ldb] : 0.0f, bneg[cb]);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = mfma_32x32x2(av[rb], bv[cb], acc[rb][cb]);
+            }
+        }
+    }
+
+    const int64_t zoff = g.part ? ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * g.sc
+                                : (int64_t)blockIdx.y * g.sc;
+    float *C = (g.part ? g.part : g.c) + zoff;
+    const bool epi = !g.part && (g.bias || g.pre || g.act || g.residual);
+    // Rows, columns and their signs derive from a lane index that the empty
+    // asm makes opaque, so that the compiler does not compute them ahead of
+    // the loop and spill.
+    int el = lane;
+    asm volatile("" : "+v"(el));
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+        const int col = col0 + 32 * (CB * wc + cb) + (el & 31);
+        if (col >= g.m) continue;
+        const float bias = epi && g.bias ? g.bias[col] : 0.0f;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int row = row0 + 32 * (RB * wr + rb) + acc_row(i, el >> 5);
+                if (row >= g.n) continue;
+                const int64_t off = (int64_t)row * g.m + col;
+                // The sign comes off by a multiplication (bits of an
+                // accumulator flipped as an integer make the compiler spill),
+                // and a zero sum stays +0.
+                float v = fmaf(acc[rb][cb][i], flip(1.0f, sign_of(row) ^ sign_of(col)), 0.0f);
+                if (epi) {
+                    // out = act(acc + bias) + residual, pre = acc + bias.
+#pragma clang fp contract(off)
+                    if (g.bias) v += bias;
+                    if (g.pre) g.pre[zoff + off] = v;
+                    if (g.act == 1) v = gelu08(v);
+                    if (g.residual) v += g.residual[zoff + off];
+                }
+                C[off] = v;
             }
         }
     }
 }
 
-// out = epilogue(sum over z of part[z]), z in order; m % 4 == 0.
+// out = epilogue(sum over z of part[z]), z in order; VEC: m % 4 == 0 and
+// 16-byte aligned operands.
+template <int V>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce(GemmArgs g, int ksplit, int64_t total)
 {
-    const int64_t n4 = total / 4;
-    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n4; q += (int64_t)gridDim.x * 256) {
-        const int64_t off = 4 * q;
-        f32x4 s = *(const f32x4 *)&g.part[off];
-        for (int z = 1; z < ksplit; ++z) {
-            const f32x4 v = *(const f32x4 *)&g.part[(int64_t)z * total + off];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] += v[c];
-        }
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const int64_t nv = total / V;
+    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < nv; q += (int64_t)gridDim.x * 256) {
+        const int64_t off = V * q;
+        vec s = *(const vec *)&g.part[off];
+        for (int z = 1; z < ksplit; ++z) s += *(const vec *)&g.part[(int64_t)z * total + off];
         if (g.bias || g.pre || g.act || g.residual) {
             const int col = (int)(off % g.m);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] = epilogue(g, s[c], off + c, col + c);
+            for (int c = 0; c < V; ++c) s[c] = epilogue(g, s[c], off + c, col + c);
         }
-        *(f32x4 *)&g.c[off] = s;
+        *(vec *)&g.c[off] = s;
     }
 }
 
@@ -550,36 +520,78 @@ int num_cus()
     return n > 0 ? n : 256;
 }
 
-template <bool TA, bool TB>
-void launch_fast(const GemmArgs &g, dim3 grid, bool split)
+template <int TM, int TN, int WR, int WC, int BK, int PER_CU, bool TWO, bool TA, bool TB>
+void launch_tiles(GemmArgs &g, int batch, int ksplit)
 {
-    // 256-row tiles when their count fills whole waves of CUs (or leaves a
-    // small tail): a 256 x 256 tile per CU reads a third less per flop, but
-    // a partly idle last wave costs more than that saves.
-    if constexpr (!TA) {
-        if (!split && g.n % 256 == 0) {
-            const int cus = num_cus();
-            const int tiles = (g.n / 256) * g.tiles_m * (int)grid.y;
-            if (tiles % cus == 0 || tiles >= 4 * cus) {
-                GemmArgs g2 = g;
-                g2.tiles_n = g.n / 256;
-                const dim3 grid2(g2.tiles_n * g2.tiles_m, grid.y, 1);
-                hipLaunchKernelGGL((gemm_f32_dma_kernel<TA, TB, false, 256>), grid2, dim3(512), 0, 0, g2);
-                return;
+    g.tiles_n = (g.n + TM - 1) / TM;
+    g.tiles_m = (g.m + TN - 1) / TN;
+    hipLaunchKernelGGL((gemm_split_kernel<TM, TN, WR, WC, BK, PER_CU, TWO, TA, TB>),
+                       dim3(g.tiles_n * g.tiles_m, batch, ksplit), dim3(64 * WR * WC), 0, 0, g);
+}
+
+// The three tiles, and what a launch with each costs: the 16-k steps of the
+// busiest CU, at the time one takes with the chip nearly empty (light_us: the
+// chain of waits of one tile) and full (full_us: throughput, and the clock
+// the power limit leaves), plus a launch's fixed cost.  Fitted to measured
+// times of 17 shapes with every tile and 1 to 8 splits (4096^3 down to
+// 17 x 33 x 5): the choice by this cost is the fastest of the measured ones
+// for 16 of them, 6 % off for one.  full_us as throughput: 256 x 256 tiles
+// 228 TFLOP/s at 4096^3 (128 x 128: 188), 128 x 128 181 TFLOP/s at
+// 8192 x 1024 x 1024 (64 x 64: 133, 256 x 256: 154); light_us: 12 products of
+// 197 x 333 x 250 11 us with 64 x 64, 17 with 128 x 128, 45 with 256 x 256.
+struct Shape {
+    int tm, tn, per_cu;
+    double full_us, light_us, fixed_us;
+};
+constexpr Shape kShapes[3] = {{256, 256, 1, 2.3, 1.75, 6.5}, {128, 128, 1, 0.73, 0.55, 4.5}, {64, 64, 3, 0.285, 0.36, 3.5}};
+constexpr int64_t kSplitBytes = int64_t(1) << 29;  // most scratch that splitting k may take
+
+template <bool TA, bool TB>
+void launch_shape(GemmArgs &g, int batch, int ksplit, int shape)
+{
+    if (shape == 0)
+        launch_tiles<256, 256, 4, 2, 16, 1, false, TA, TB>(g, batch, ksplit);
+    else if (shape == 1)
+        launch_tiles<128, 128, 4, 2, 32, 1, true, TA, TB>(g, batch, ksplit);
+    else
+        launch_tiles<64, 64, 2, 2, 32, 3, true, TA, TB>(g, batch, ksplit);
+}
+
+// k per split for `want` splits, a multiple of every tile's slab.
+int split_chunk(int k, int want)
+{
+    return ((k + want - 1) / want + 31) / 32 * 32;
+}
+
+// The cheapest tile and number of k splits.
+void choose_shape(const GemmArgs &g, int batch, int &shape, int &ksplit)
+{
+    const double cus = num_cus(), total = (double)batch * g.n * g.m;
+    double best = INFINITY;
+    for (int s = 0; s < 3; ++s) {
+        const Shape &p = kShapes[s];
+        const double tiles = (double)((g.n + p.tm - 1) / p.tm) * ((g.m + p.tn - 1) / p.tn) * batch;
+        for (int want : {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48, 64}) {
+            if (want > 1 && (g.k / want < 64 || 4 * want * total > kSplitBytes)) break;
+            // The 256 x 256 tile sums all six part products together, the
+            // others keep the small ones apart and err a third as much: it
+            // splits k only as often as fills the chip, with short sums.
+            if (s == 0 && want > 1 && (want + 1) * tiles <= cus) continue;
+            const int chunk = want > 1 ? split_chunk(g.k, want) : g.k;
+            const int splits = want > 1 ? (g.k + chunk - 1) / chunk : 1;
+            const double work = tiles * splits, rounds = ceil(work / cus), steps = (chunk + 15) / 16;
+            const double step_us = p.per_cu > 1
+                                       ? fmax(p.light_us, p.full_us * rounds)
+                                       : rounds * (p.light_us + (p.full_us - p.light_us) * fmin(1.0, work / cus));
+            double us = p.fixed_us + steps * step_us;
+            if (splits > 1) us += 3.0 + (2 * splits + 1) * 4 * total / 5e6;  // the reduction's launch and bytes
+            if (us < best) {
+                best = us;
+                shape = s;
+                ksplit = splits;
             }
         }
     }
-    if (split) {
-        hipLaunchKernelGGL((gemm_f32_dma_kernel<TA, TB, true>), grid, dim3(kThreads), 0, 0, g);
-        return;
-    }
-    // No more tiles than CUs: one workgroup per CU either way, so give it two
-    // k groups (two waves per SIMD); needs an even slab count.
-    if ((int)(grid.x * grid.y) <= num_cus() && (g.k / FK) % 2 == 0 && g.k >= 4 * FK) {
-        hipLaunchKernelGGL((gemm_f32_dma_kernel<TA, TB, false, FM, 2>), grid, dim3(2 * kThreads), 0, 0, g);
-        return;
-    }
-    hipLaunchKernelGGL((gemm_f32_dma_kernel<TA, TB, false>), grid, dim3(kThreads), 0, 0, g);
 }
 
 int gemm_launch(const float *a, const float *b, float *out, int batch, int n, int m, int k,
@@ -590,8 +602,9 @@ int gemm_launch(const float *a, const float *b, float *out, int batch, int n, in
     if ((int64_t)n * m == 0 || batch == 0) return EMBER_OK;
     // k == 0: a and b are empty (null from alloc_memory(0)) and every output
     // is an empty sum, i.e. 0 before the epilogue, as in the reference's CPU
-    // loop; the generic kernel below never reads a or b then.
+    // loop; the kernel never reads a or b then.
     if (!out || (k > 0 && (!a || !b))) return record_error(EMBER_ERR_INVALID_ARGUMENT, who);
+    if (batch > 65535) return record_error(EMBER_ERR_UNSUPPORTED, who);
     GemmArgs g;
     g.a = a;
     g.b = b;
@@ -606,65 +619,39 @@ int gemm_launch(const float *a, const float *b, float *out, int batch, int n, in
     g.sa = (int64_t)n * k;
     g.sb = (int64_t)k * m;
     g.sc = (int64_t)n * m;
-    g.tiles_n = (n + BM - 1) / BM;
-    g.tiles_m = (m + BN - 1) / BN;
     g.kchunk = k;
     g.part = nullptr;
     g.bias = bias;
     g.residual = residual;
     g.pre = pre;
     g.act = act;
-    if (batch > 65535) return record_error(EMBER_ERR_UNSUPPORTED, who);
-    const bool vec = (k % 4 == 0) && (m % 4 == 0) && (n % 4 == 0 || !ta) &&
-                     (((uintptr_t)a | (uintptr_t)b) % 16 == 0);
-    // The fast kernel moves out, pre and residual as 16-byte vectors, and
-    // addresses a tile's rows with 32-bit byte offsets (row pitch < 2^22).
-    if (vec && n % FM == 0 && m % FN == 0 && k % FK == 0 && k > 0 && g.lda < (1 << 22) &&
-        g.ldb < (1 << 22) &&
-        (((uintptr_t)out | (uintptr_t)pre | (uintptr_t)residual) % 16) == 0) {
-        g.tiles_n = n / FM;
-        g.tiles_m = m / FN;
-        const int work = g.tiles_n * g.tiles_m * batch;
-        // Fewer tiles than CUs: split k so that about two workgroups run per
-        // CU, each over at least 512 of k.
-        int ksplit = 1;
-        const int cus = num_cus();
-        if (work < cus && k >= 1024) {
-            ksplit = min(2 * cus / work, k / 512);
-            if (ksplit > 64) ksplit = 64;
-            if (ksplit > 1) {
-                g.kchunk = ((k + ksplit - 1) / ksplit + FK - 1) / FK * FK;
-                ksplit = (k + g.kchunk - 1) / g.kchunk;
-            }
-        }
-        dim3 grid(g.tiles_n * g.tiles_m, batch, ksplit);
-        const bool split = ksplit > 1;
-        if (split) {
-            const int64_t total = (int64_t)batch * n * m;
-            g.part = (float *)scratch(kScratchGemmSplit, (size_t)ksplit * total * sizeof(float));
-            if (!g.part) return EMBER_ERR_OUT_OF_MEMORY;
-        }
-        if (ta)
-            tb ? launch_fast<true, true>(g, grid, split) : launch_fast<true, false>(g, grid, split);
+
+    int shape = 2, ksplit = 1;
+    choose_shape(g, batch, shape, ksplit);
+    const int64_t total = (int64_t)batch * n * m;
+    if (ksplit > 1) {
+        g.part = (float *)scratch(kScratchGemmSplit, (size_t)ksplit * total * sizeof(float), true);
+        if (g.part)
+            g.kchunk = split_chunk(k, ksplit);
         else
-            tb ? launch_fast<false, true>(g, grid, split) : launch_fast<false, false>(g, grid, split);
-        if (!launch_ok(who)) return EMBER_ERR_DEVICE;
-        if (split) {
-            const int64_t total = (int64_t)batch * n * m;
-            int64_t blocks = (total / 4 + 255) / 256;
-            if (blocks > 8 * cus) blocks = 8 * cus;
-            hipLaunchKernelGGL(gemm_splitk_reduce, dim3((unsigned)blocks), dim3(256), 0, 0, g,
-                               ksplit, total);
-            if (!launch_ok("gemm_splitk_reduce")) return EMBER_ERR_DEVICE;
-        }
-        return EMBER_OK;
+            ksplit = 1;  // no memory for the parts: one sum per element
     }
-    const dim3 grid(g.tiles_n * g.tiles_m, batch);
-    if (vec)
-        hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, dim3(kThreads), 0, 0, g);
+    if (ta)
+        tb ? launch_shape<true, true>(g, batch, ksplit, shape) : launch_shape<true, false>(g, batch, ksplit, shape);
     else
-        hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, dim3(kThreads), 0, 0, g);
-    return launch_ok(who) ? EMBER_OK : EMBER_ERR_DEVICE;
+        tb ? launch_shape<false, true>(g, batch, ksplit, shape) : launch_shape<false, false>(g, batch, ksplit, shape);
+    if (!launch_ok(who)) return EMBER_ERR_DEVICE;
+    if (ksplit > 1) {
+        const bool vec = m % 4 == 0 && ((uintptr_t)out | (uintptr_t)pre | (uintptr_t)residual | (uintptr_t)bias) % 16 == 0;
+        int64_t blocks = (total / (vec ? 4 : 1) + 255) / 256;
+        if (blocks > 8 * num_cus()) blocks = 8 * num_cus();
+        if (vec)
+            hipLaunchKernelGGL(gemm_splitk_reduce<4>, dim3((unsigned)blocks), dim3(256), 0, 0, g, ksplit, total);
+        else
+            hipLaunchKernelGGL(gemm_splitk_reduce<1>, dim3((unsigned)blocks), dim3(256), 0, 0, g, ksplit, total);
+        if (!launch_ok("gemm_splitk_reduce")) return EMBER_ERR_DEVICE;
+    }
+    return EMBER_OK;
 }
 
 }  // namespace

@@ -96,7 +96,7 @@ ScratchBuf g_scratch[kMaxDevices][kScratchSlots];
 std::mutex g_scratch_mu;
 }  // namespace
 
-void *scratch(int slot, size_t bytes)
+void *scratch(int slot, size_t bytes, bool optional)
 {
     int dev = 0;
     if (!hip_ok(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
@@ -116,7 +116,12 @@ void *scratch(int slot, size_t bytes)
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
     void *p = nullptr;
-    if (!hip_ok(hipMalloc(&p, want), "hipMalloc(scratch)")) return nullptr;
+    const hipError_t err = hipMalloc(&p, want);
+    if (err == hipErrorOutOfMemory && optional) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (!hip_ok(err, "hipMalloc(scratch)")) return nullptr;
     s.ptr = p;
     s.bytes = want;
     return p;

@@ -1,0 +1,129 @@
+"""The split-bf16 GEMM where it can go wrong: tile edges and short last k-slabs
+of each tile shape and orientation, operands that do not start on 16 bytes,
+values the split cannot carry (infinities, NaN, magnitudes next to the largest
+float, rows below 2^-100), and its error against float64 next to the fp32
+chain's."""
+
+import numpy as np
+import pytest
+
+import gpu_helpers as G
+from ember_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _u(shape, seed):
+    return np.random.default_rng(seed).uniform(-1, 1, shape).astype(np.float32)
+
+
+def _stored(x, trans):
+    return np.ascontiguousarray(x.T) if trans else x
+
+
+def _bound(a, b):
+    """6 roundings per 16 products of partial sums of at most |a||b|, and the
+    part products left out (2^-25 of |a||b|)."""
+    k = a.shape[1]
+    mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    return (0.375 * k + 8) * 2.0 ** -24 * mag + 2.0 ** -25 * mag
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("n,k,m", [
+    (1, 1, 1), (64, 32, 64), (65, 33, 63), (63, 31, 65), (3, 64, 200),     # 64 x 64 tiles, one to two slabs
+    (129, 1030, 127), (640, 97, 1537),                                     # splits; ragged in all three
+    (2500, 130, 1900), (4096, 15, 4097), (4097, 47, 4095),                 # 128 and 256 tiles with remainders
+])
+def test_shapes_and_orientations(n, k, m, ta, tb):
+    a, b = _u((n, k), n + k), _u((k, m), m)
+    got = G.gemm_ex(_stored(a, ta), _stored(b, tb), ta, tb)
+    rows = np.unique(np.r_[0, n - 1, np.random.default_rng(0).integers(0, n, 40)])
+    ref = a[rows].astype(np.float64) @ b.astype(np.float64)
+    assert (np.abs(got[rows] - ref) <= _bound(a[rows], b)).all()
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_operands_off_16_bytes(offset):
+    n, k, m = 70, 100, 130
+    a, b = _u((n, k), 1), _u((k, m), 2)
+    bufs = [capi.DeviceArray((x.size + 4,), np.r_[np.zeros(offset, np.float32), x.ravel(),
+                                                  np.zeros(4 - offset, np.float32)]) for x in (a, b)]
+    out = capi.DeviceArray((n * m + 4,))
+    L = capi.lib()
+    L.matmul(bufs[0].ptr + 4 * offset, bufs[1].ptr + 4 * offset, out.ptr + 4 * offset, n, m, k)
+    capi.check(what="matmul")
+    got = out.numpy()[offset:offset + n * m].reshape(n, m)
+    assert (np.abs(got - a.astype(np.float64) @ b) <= _bound(a, b)).all()
+
+
+@pytest.mark.parametrize("n,k,m", [(100, 70, 90), (600, 500, 700), (4096, 40, 4096)])
+def test_infinities_and_nan_follow_ieee(n, k, m):
+    """An infinite element gives +-inf or NaN exactly where fp32 products and
+    sums do, and leaves every other element as it is."""
+    a, b = _u((n, k), 3), _u((k, m), 4)
+    a[n // 2, 3], a[n - 1, k - 1], b[5, m // 3] = np.inf, -np.inf, -np.inf
+    b[3, 7] = 0.0          # inf * 0
+    a[1, 2] = np.nan
+    with np.errstate(invalid="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = G.gemm_ex(a, b)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
+    ok = np.isfinite(ref)
+    fa, fb = np.where(np.isfinite(a), a, 0), np.where(np.isfinite(b), b, 0)
+    assert (np.abs(got - ref)[ok] <= _bound(fa, fb)[ok]).all()
+
+
+def test_magnitudes_next_to_the_largest_float():
+    """The largest finite floats round up to infinity in bf16; their products
+    with small factors are finite."""
+    n, k, m = 80, 48, 70
+    a, b = _u((n, k), 5), _u((k, m), 6) * np.float32(2.0 ** -20)
+    a[4] = np.finfo(np.float32).max
+    a[9, :] = np.finfo(np.float32).min
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    assert (np.abs(G.gemm_ex(a, b) - ref) <= _bound(a, b)).all()
+
+
+@pytest.mark.parametrize("exponent", [-99, -101, -110, -125])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_tiny_rows_keep_their_precision(exponent, ta, tb):
+    """Rows of a and columns of b below what three bf16 parts can hold; the
+    other operand brings the results back into range."""
+    n, k, m = 90, 200, 75
+    a, b = _u((n, k), 7), _u((k, m), 8) * np.float32(2.0 ** 60)
+    a[10:20] *= np.float32(2.0 ** exponent)
+    b[:, 30] *= np.float32(2.0 ** (exponent - 60))
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = G.gemm_ex(_stored(a, ta), _stored(b, tb), ta, tb)
+    err, bound = np.abs(got - ref), _bound(a, b) + 2.0 ** -149 * k
+    assert (err <= bound).all()
+
+
+@pytest.mark.parametrize("n,k,m,fp32_chain", [(4096, 1024, 4096, 5.7e-7), (1024, 8192, 1024, 4.1e-7),
+                                               (8192, 1024, 1024, 4.0e-7), (197, 333, 250, 3.2e-7)])
+def test_error_no_larger_than_the_fp32_instructions(n, k, m, fp32_chain):
+    """Relative 2-norm error against float64, U(-1, 1) operands: below what
+    the kernels on the fp32 matrix instruction measured at these shapes."""
+    a, b = _u((n, k), 9), _u((k, m), 10)
+    got = G.gemm_ex(a, b)
+    rows = np.arange(0, n, max(1, n // 64))
+    ref = a[rows].astype(np.float64) @ b.astype(np.float64)
+    assert np.linalg.norm(got[rows] - ref) / np.linalg.norm(ref) <= fp32_chain
+
+
+@pytest.mark.parametrize("n,k,m,fp32_chain", [(4096, 1024, 1024, 5.5e-7), (4096, 4096, 4096, 1.12e-6), (1024, 8192, 512, 4.5e-7)])
+def test_sums_over_rows_and_columns_are_unbiased(n, k, m, fp32_chain):
+    """A rounding of one direction in the matrix core would add up over the
+    rows of a column (a bias gradient): held to what the fp32 instruction's
+    sums measured (1.3e-5 without the row and column signs at 4096^3)."""
+    a, b = _u((n, k), 11), _u((k, m), 12)
+    got = G.gemm_ex(a, b).astype(np.float64)
+    for axis, ref in ((0, a.sum(0, dtype=np.float64) @ b), (1, a.astype(np.float64) @ b.sum(1, dtype=np.float64))):
+        assert np.linalg.norm(got.sum(axis) - ref) / np.linalg.norm(ref) <= 1.2 * fp32_chain
+
+
+def test_zero_products_give_positive_zero():
+    a, b = _u((70, 40), 13), np.zeros((40, 90), np.float32)
+    assert not np.signbit(G.gemm_ex(a, b)).any()
