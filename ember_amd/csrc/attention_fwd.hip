@@ -4,38 +4,36 @@
 // new, slotted beside matmul in src/tensor/operators.h:20-27.  Its semantics
 // are those of oracle/ember_oracle.c (oracle_attention_fwd).
 //
-// Work decomposition.  One workgroup = 4 waves = 128 queries of one (b, h);
-// each wave owns 32 queries for the whole kernel.  The workgroup walks the
-// keys in tiles of 64: every tile of K and V is read from HBM once and
-// staged in LDS, where the 4 waves share it.  The copies go HBM -> LDS
-// directly (buffer_load_dwordx4 ... lds, no registers) and overlap the
-// products: V of tile t lands while S of tile t is computed, K of tile t+1
-// while V of tile t is multiplied; two barriers per tile.
-// Short sequences (S <= 64, HBM-bound) use one wave per 32-query block
-// instead, with no barriers (attn_fwd_wave, D >= 64), or pack heads
-// (attn_fwd_packed, D = 32): S <= 32 puts 4 heads in a workgroup (one per
-// wave, tiles of 32 keys) and S <= 64 puts 2 (two waves each), so that no
-// wave idles and every wave keeps loading.
-// 64 < S <= 96, and causal S <= 128, at D >= 64 take attn_fwd_wave with one
-// wave per pair of query blocks.
+// S > 64 in general: attention_fwd_tiles.hip (attn_fwd_kernel, on the bf16
+// matrix cores at fp32 precision).  This file has the kernels for the shapes
+// that one fills badly, all on v_mfma_f32_32x32x2f32 (or 16x16x4):
+//   few heads of moderate length   attn_fwd_split, attn_fwd_split16: the keys
+//                                  split across a workgroup's waves
+//   S <= 64, HBM-bound             attn_fwd_wave (D >= 64): one wave per
+//                                  32-query block, no barriers;
+//                                  attn_fwd_packed (D = 32): 2 or 4 heads
+//                                  per workgroup
+//   64 < S <= 128 (D >= 64)        attn_fwd_head, or attn_fwd_wave with one
+//                                  wave per pair of query blocks
 //
-// Per tile and wave (all products on v_mfma_f32_32x32x2f32):
-//   S^T (64 keys x 32 queries) = K_tile . Q^T   -- K from LDS, Q^T resident in
-//                                                  registers for the kernel
+// Per tile and wave:
+//   S^T (keys x 32 queries) = K . Q^T     -- Q^T resident in registers
 //   online softmax over keys: each lane holds one query column, so the row
-//   max is an in-lane max over 32 registers plus one exchange with lane^32,
-//   and the row sum stays a per-lane partial until the end
-//   O^T (D x 32 queries) += V_tile^T . P^T      -- P^T straight from the S^T
-//                                                  accumulator registers
+//   max is an in-lane max plus one exchange with lane^32, and the row sum
+//   stays a per-lane partial until the end
+//   O^T (D x 32 queries) += V^T . P^T     -- P^T straight from the S^T
+//                                            accumulator registers
 // The softmax runs in base 2 with scale*log2(e) folded into one FMA per
-// score, on v_exp_f32, with lazy rescaling of O (see the loop); LSE is
-// stored in natural log.  Causal: tiles wholly above a wave's
-// diagonal are skipped per wave, the mask (key <= query, integer compare) is
-// applied only on tiles that cross the diagonal or the sequence end.
+// score, on v_exp_f32.  Lazy rescaling: the reference max is raised, and O
+// rescaled, only when some lane's scores would otherwise exceed it by more
+// than 2^8.  LSE is stored in natural log.  The causal mask (key <= query, an
+// integer compare) is applied only on tiles that cross the diagonal or the
+// sequence end; tiles wholly above it are skipped.
 #include <math.h>
 
 #include <type_traits>
 
+#include "attention_fwd.h"
 #include "common.h"
 #include "lds_dma.h"
 #include "mfma.h"
@@ -48,319 +46,6 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kBr = 32 * kWaves;  // queries per workgroup (one head per workgroup)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-
-struct FwdArgs {
-    const float *q, *k, *v;
-    float *o, *lse;
-    int H, S, nqb, nbh;
-    float c;  // scale * log2(e)
-    int64_t in_sb, in_sh, in_ss, out_sb, out_sh, out_ss;
-};
-
-// Copy layout of one 64-key tile for the direct HBM -> LDS copies.  A copy is
-// 64 lanes x 16 bytes = 1 KiB of LDS; copy t of a tile fills 16-byte chunks
-// 64t .. 64t+63.  K rows are padded to D+4 floats (conflict-free reads of a
-// column of chunks by 32 lanes): a padding chunk re-reads the tile's first
-// chunk (valid memory, never used).  V rows are dense.
-template <int D> struct FwdTile {
-    static constexpr int KSTR = D + 4;                       // floats per K row
-    static constexpr int KCH = KSTR / 4;                     // chunks per K row
-    static constexpr int KCOP = KCH;                         // copies per K tile: 64 rows * KCH / 64
-    static constexpr int VCOP = D / 4;                       // copies per V tile
-    static constexpr int KSL = (KCOP + kWaves - 1) / kWaves; // K copy slots per wave
-    static constexpr int VSL = VCOP / kWaves;                // V copy slots per wave
-    static constexpr int VROWS = kWaves * 256 / D;           // V rows between a wave's slots
-};
-
-// One head per workgroup, S > 64 (see the file comment).  Per tile t:
-//   wait for this wave's K copies, barrier (K(t) complete, Vs free)
-//   copy V(t) -> Vs;  S^T = K . Q^T;  mask, softmax
-//   wait for this wave's V copies, barrier (V(t) complete, Ks free)
-//   copy K(t+1) -> Ks;  O^T += V^T . P^T
-// A wave whose queries all precede the tile (causal) skips the products
-// but still issues its copies and meets both barriers.
-// Workgroups per CU: two, or three at D = 64 (LDS fits three there; the
-// causal D = 64 kernel fits three in registers thanks to its split loop,
-// see the end of the kernel).
-template <int D, bool CAUSAL, bool PAIRQ>
-__global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_fwd_kernel(FwdArgs a)
-{
-    typedef FwdTile<D> T;
-    constexpr int DH = D / 2;   // contraction length per lane half (k-steps)
-    constexpr int DB = D / 32;  // 32-row blocks of O^T
-    constexpr int KSTR = T::KSTR;
-    constexpr int kBc = 64;
-    // D = 128 keeps one offset register per V copy slot (it has the
-    // registers, and it saves the per-slot descriptor arithmetic); smaller D
-    // keeps one and moves the descriptor base per slot.
-    constexpr bool kVoffRegs = D == 128;
-    __shared__ float Ks[kBc * KSTR];
-    __shared__ float Vs[kBc * D];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h32 = lane >> 5;
-    const int l32 = lane & 31;
-
-    // Heavy (late) query blocks first so the causal triangle load-balances.
-    // PAIRQ (causal): the workgroup takes query blocks nqb - 1 - p and p of
-    // its head, one after the other: 2 (nqb + 1) key tiles for every
-    // workgroup (the middle block of an odd nqb alone, dispatched last).
-    const int per_head = PAIRQ ? (a.nqb + 1) / 2 : a.nqb;
-    const int BH = (int)(gridDim.x / per_head);
-    const int qbr = blockIdx.x / BH;
-    const int bh = blockIdx.x - qbr * BH;
-    const int qb_first = CAUSAL ? (a.nqb - 1 - qbr) : qbr;
-    const int b = bh / a.H;
-    const int hh = bh - b * a.H;
-    const int S = a.S;
-    const int64_t in_base = (int64_t)b * a.in_sb + (int64_t)hh * a.in_sh;
-    const int in_ss = (int)a.in_ss;  // < 2^24 (checked on the host)
-    const float *__restrict__ kbase = a.k + in_base;
-    const float *__restrict__ vbase = a.v + in_base;
-
-    // Byte offsets of this wave's copy slots within a tile (slot s is copy
-    // t = w + 4s, chunk p = 64t + lane).  The element offset r * in_ss + 4c
-    // (r < 64, in_ss < 2^24) fits an int; the byte offset, up to
-    // 4 * 63 * 2^24 + 4 * D, only fits 32 bits unsigned.
-    unsigned koff[T::KSL];
-#pragma unroll
-    for (int s = 0; s < T::KSL; ++s) {
-        const int p = 64 * (w + kWaves * s) + lane;
-        const int r = p / T::KCH, c = p - r * T::KCH;
-        koff[s] = c < D / 4 ? 4u * (unsigned)(r * in_ss + 4 * c) : 0u;
-    }
-    unsigned voff[kVoffRegs ? T::VSL : 1];
-#pragma unroll
-    for (int s = 0; s < (kVoffRegs ? T::VSL : 1); ++s) {
-        const int p = 64 * (w + kWaves * s) + lane;
-        const int r = p / (D / 4), c = p - r * (D / 4);
-        voff[s] = 4u * (unsigned)(r * in_ss + 4 * c);
-    }
-
-    // Rows past the sequence end re-read row S-1: their scores are masked,
-    // so they contribute exactly 0.  On that (last) tile the offsets are
-    // recomputed from an opaque lane index, so that the compiler does not
-    // keep a second set live across the loop.
-    auto fetch_k = [&](int n0) {
-        const __amdgpu_buffer_rsrc_t src = dma_rsrc(kbase + (int64_t)n0 * in_ss);
-        const int rmax = S - 1 - n0;
-        if (rmax >= kBc - 1) {
-#pragma unroll
-            for (int s = 0; s < T::KSL; ++s)
-                if (w + kWaves * s < T::KCOP) dma16_buf(src, koff[s], Ks + 256 * (w + kWaves * s));
-        } else {
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-#pragma unroll
-            for (int s = 0; s < T::KSL; ++s) {
-                const int t = w + kWaves * s;
-                if (t < T::KCOP) {
-                    const int p = 64 * t + ln;
-                    const int r = p / T::KCH, c = p - r * T::KCH;
-                    const unsigned off = c < D / 4 ? 4u * (unsigned)(min(r, rmax) * in_ss + 4 * c) : 0u;
-                    dma16_buf(src, off, Ks + 256 * t);
-                }
-            }
-        }
-    };
-    auto fetch_v = [&](int n0) {
-        const int rmax = S - 1 - n0;
-        if (rmax >= kBc - 1) {
-#pragma unroll
-            for (int s = 0; s < T::VSL; ++s) {
-                if constexpr (kVoffRegs)
-                    dma16_buf(dma_rsrc(vbase + (int64_t)n0 * in_ss), voff[s],
-                              Vs + 256 * (w + kWaves * s));
-                else
-                    dma16_buf(dma_rsrc(vbase + (int64_t)(n0 + T::VROWS * s) * in_ss), voff[0],
-                              Vs + 256 * (w + kWaves * s));
-            }
-        } else {
-            const __amdgpu_buffer_rsrc_t src = dma_rsrc(vbase + (int64_t)n0 * in_ss);
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-#pragma unroll
-            for (int s = 0; s < T::VSL; ++s) {
-                const int t = w + kWaves * s;
-                const int p = 64 * t + ln;
-                const int r = p / (D / 4), c = p - r * (D / 4);
-                dma16_buf(src, 4u * (unsigned)(min(r, rmax) * in_ss + 4 * c), Vs + 256 * t);
-            }
-        }
-    };
-
-    // Query block qb; K tile 0 already requested unless first; next: a
-    // second block follows (its K tile 0, the same head's, is requested
-    // during this block's last tile).
-    auto run_block = [&](int qb, bool first, bool next) {
-    const int q0 = qb * kBr;
-    const int m0 = q0 + 32 * w;
-    const int mq = m0 + l32;
-    const int kend = CAUSAL ? min(S, q0 + kBr) : S;
-    const int ntiles = (kend + kBc - 1) / kBc;
-    if (first) fetch_k(0);
-
-    // Q^T operand: lane holds Q[mq][h32*DH + kk] for k-step kk.
-    float qr[DH];
-    {
-        const int mrow = mq < S ? mq : S - 1;
-        const float *src = a.q + in_base + (int64_t)mrow * a.in_ss + h32 * DH;
-#pragma unroll
-        for (int kk = 0; kk < DH; kk += 4) {
-            f32x4 t = *(const f32x4 *)(src + kk);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) qr[kk + j] = t[j];
-        }
-    }
-
-    f32x16 oacc[DB];
-#pragma unroll
-    for (int db = 0; db < DB; ++db) oacc[db] = zero16();
-    float mrun = -INFINITY;  // reference max of s*c for query mq (see below)
-    float lrun = 0.0f;       // this lane half's share of the running sum
-
-    auto tile = [&](int t, auto masked) {
-        constexpr bool MASKED = decltype(masked)::value;
-        const int n0 = t * kBc;
-        wait_vmem();      // this wave's copies of K tile t have landed
-        __syncthreads();  // all of K tile t is in LDS; every wave is done with Vs
-        fetch_v(n0);
-        const bool active = !MASKED || !(CAUSAL && n0 > m0 + 31);  // some key at or before a query
-        f32x16 sacc[kBc / 32];
-        if (active) {
-            // S^T = K . Q^T for two 32-key blocks.
-#pragma unroll
-            for (int blk = 0; blk < kBc / 32; ++blk) sacc[blk] = zero16();
-#pragma unroll
-            for (int kk = 0; kk < DH; kk += 4) {
-#pragma unroll
-                for (int blk = 0; blk < kBc / 32; ++blk) {
-                    const f32x4 kf = *(const f32x4 *)&Ks[(32 * blk + l32) * KSTR + h32 * DH + kk];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) sacc[blk] = mfma_32x32x2(kf[j], qr[kk + j], sacc[blk]);
-                }
-            }
-
-            // Mask (diagonal and tail tiles only), tile max of the raw scores.
-            const bool need_mask = MASKED && ((n0 + kBc > S) || (CAUSAL && n0 + kBc - 1 > m0));
-            if (need_mask) {
-#pragma unroll
-                for (int blk = 0; blk < kBc / 32; ++blk) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int n = n0 + 32 * blk + acc_row(i, h32);
-                        const bool vis = (n < S) & (!CAUSAL | (n <= mq));
-                        sacc[blk][i] = vis ? sacc[blk][i] : -INFINITY;
-                    }
-                }
-            }
-            float tmax = -INFINITY;
-#pragma unroll
-            for (int blk = 0; blk < kBc / 32; ++blk)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, sacc[blk][i]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-            // Scaled tile max (scale >= 0, checked on the host).  The
-            // reference max mrun is raised only when some lane's scores would
-            // otherwise exceed it by more than 2^8 (lazy rescaling): the
-            // result is the same softmax, and most tiles skip the rescale of
-            // O.  Tile 0 holds key 0, visible to every query, so it always
-            // sets a finite mrun.
-            const float tm2 = tmax * a.c;
-            if (__ballot(tm2 > mrun + 8.0f) != 0) {
-                const float mnew = fmaxf(mrun, tm2);
-                const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
-                mrun = mnew;
-                lrun *= alpha;
-#pragma unroll
-                for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
-            }
-            if (need_mask) {
-#pragma unroll
-                for (int blk = 0; blk < kBc / 32; ++blk) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float sv = sacc[blk][i];
-                        const float p = sv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(sv, a.c, -mrun));
-                        sacc[blk][i] = p;
-                        lrun += p;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int blk = 0; blk < kBc / 32; ++blk) {
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const float p = __builtin_amdgcn_exp2f(fmaf(sacc[blk][i], a.c, -mrun));
-                        sacc[blk][i] = p;
-                        lrun += p;
-                    }
-                }
-            }
-        }
-        wait_vmem();      // this wave's copies of V tile t have landed
-        __syncthreads();  // all of V tile t is in LDS; every wave is done with Ks
-        if (t + 1 < ntiles)
-            fetch_k(n0 + kBc);
-        else if (next)
-            fetch_k(0);
-        if (active) {
-            // O^T += V^T . P^T; lane l32 covers O^T rows d = DB*l32 + db.
-#pragma unroll
-            for (int blk = 0; blk < kBc / 32; ++blk) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int nr = 32 * blk + acc_row(i, h32);
-                    const typename VecN<DB>::T vf = *(const typename VecN<DB>::T *)&Vs[nr * D + DB * l32];
-#pragma unroll
-                    for (int db = 0; db < DB; ++db)
-                        oacc[db] = mfma_32x32x2(vget<DB>(vf, db), sacc[blk][i], oacc[db]);
-                }
-            }
-        }
-    };
-    // Causal D = 64: the tiles wholly before the workgroup's first query need
-    // no mask for any wave and run a mask-free copy of the loop body; with
-    // only the last (diagonal) tiles carrying the mask the kernel fits three
-    // workgroups per CU without spilling (146 VGPRs; one loop with the mask
-    // test inside needed 178, or spilled 8-10 at three per CU).  Measured:
-    // +1 % at config 2, +3 % at S = 4096.  The other instantiations keep one
-    // loop (splitting measured -1 % at D = 128 and -2 % for non-causal D = 64).
-    int t = 0;
-    if constexpr (D == 64 && CAUSAL) {
-        for (const int nfull = min(q0 / kBc, ntiles); t < nfull; ++t) tile(t, std::false_type{});
-    }
-    for (; t < ntiles; ++t) tile(t, std::true_type{});
-
-    const float ltot = lrun + __shfl_xor(lrun, 32);
-    if (mq < S) {
-        const float inv = 1.0f / ltot;
-        float *orow = a.o + (int64_t)b * a.out_sb + (int64_t)hh * a.out_sh + (int64_t)mq * a.out_ss;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int r = acc_row(i, h32);  // O^T row block index -> d = DB*r + db
-            typename VecN<DB>::T outv;
-            if constexpr (DB == 1) {
-                outv = oacc[0][i] * inv;
-            } else {
-#pragma unroll
-                for (int db = 0; db < DB; ++db) outv[db] = oacc[db][i] * inv;
-            }
-            *(typename VecN<DB>::T *)(orow + DB * r) = outv;
-        }
-        if (h32 == 0) a.lse[(int64_t)bh * S + mq] = (mrun + log2f(ltot)) * kLn2;
-    }
-    };
-    if constexpr (PAIRQ) {
-        const int second = a.nqb - 1 - qb_first;
-        run_block(qb_first, true, second != qb_first);
-        if (second != qb_first) run_block(second, false, false);
-    } else {
-        run_block(qb_first, true, false);
-    }
-}
 
 // S <= 64 (D = 64 and 128, see launch_fwd): one
 // wave per (head, 32-query block), four independent
@@ -1458,27 +1143,7 @@ int launch_fwd(FwdArgs args, int64_t nbh)
             return launch_ok("attn_fwd_wave_pair") ? EMBER_OK : EMBER_ERR_DEVICE;
         }
     }
-    if (args.S > 64) {
-        args.nqb = (args.S + kBr - 1) / kBr;
-        // Causal launches whose block pairs all fit one round of resident
-        // workgroups take the blocks in pairs of equal work (no tail of
-        // light blocks): measured +15-24 % at B2-B4 H16 S = 1024-2048, +0.6 %
-        // at B8 H16 S = 1024 D = 64.  Larger ones keep single blocks, heavy
-        // first (pairs there measured -0.6 to -2 %).
-        if constexpr (CAUSAL) {
-            const int ncu = device_cu_count();
-            const int64_t slots = (int64_t)(ncu > 0 ? ncu : 256) * (D == 64 ? 3 : 2);
-            const int64_t pairs = (int64_t)(args.nqb + 1) / 2 * nbh;
-            if (args.nqb >= 4 && pairs <= slots) {
-                hipLaunchKernelGGL((attn_fwd_kernel<D, CAUSAL, true>), dim3((unsigned)pairs), dim3(kThreads), 0, 0,
-                                   args);
-                return launch_ok("attn_fwd_kernel_pairs") ? EMBER_OK : EMBER_ERR_DEVICE;
-            }
-        }
-        const int nblocks = args.nqb * (int)nbh;
-        hipLaunchKernelGGL((attn_fwd_kernel<D, CAUSAL, false>), dim3(nblocks), dim3(kThreads), 0, 0, args);
-        return launch_ok("attn_fwd_kernel") ? EMBER_OK : EMBER_ERR_DEVICE;
-    }
+    if (args.S > 64) return launch_fwd_tiles(args, D, CAUSAL);
     // S <= 64: the wave kernel at D = 128 (4.7 TB/s at S = 32 and 4.0 at
     // S = 64, where the packed kernel moves 3.8 and 2.9) and at D = 64
     // (against the packed kernel: causal +9-13 % at S = 32, +25 % at S = 48,

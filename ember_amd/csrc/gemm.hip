@@ -60,11 +60,6 @@ __device__ __forceinline__ float epilogue(const GemmArgs &g, float v, int64_t of
     return v;
 }
 
-__device__ __forceinline__ bool is_tiny(float m)
-{
-    return m > 0.0f && m < kSplitTiny;
-}
-
 // One operand's share of a k-slab: R tile rows (rows of a, columns of b) by
 // BK of k, loaded into registers by NT threads, split, and stored to LDS as
 // three bf16 planes.  A thread holds G groups of 8 consecutive k of one row.
@@ -89,7 +84,7 @@ struct Operand {
     unsigned voff;      // !KC: this lane's byte offset from there
     int kq[G];          // the group's k offset within the slab
     float v[G][8];
-    float big[G];       // largest magnitude the group's row has shown
+    unsigned bits[G];   // OR of the group's elements so far (split_tiny)
     unsigned neg[G];    // sign_of the group's row
     unsigned s[G][3][2];  // two split pairs: hi, mid, lo
 
@@ -121,7 +116,7 @@ struct Operand {
             neg[g] = sign_of(row0 + row_of(tid, g));
             p[g] = KC ? base + (int64_t)(row0 + r) * ld + kbeg + 8 * q : base + (int64_t)(kbeg + 8 * q) * ld + row0;
             if (!KC) voff = 4u * (unsigned)r;
-            big[g] = 0.0f;
+            bits[g] = 0;
         }
     }
     __device__ __forceinline__ float at(int g, int j, int64_t ld) const
@@ -166,7 +161,7 @@ struct Operand {
     __device__ __forceinline__ void split_store(int g, int i, u32x4 *__restrict__ lds, int tid)
     {
         const float x = flip(v[g][2 * i], neg[g]), y = flip(v[g][2 * i + 1], neg[g]);
-        big[g] = fmaxf(big[g], fmaxf(fabsf(x), fabsf(y)));
+        bits[g] |= float_bits(v[g][2 * i]) | float_bits(v[g][2 * i + 1]);
         split_pair(x, y, s[g][0][i & 1], s[g][1][i & 1], s[g][2][i & 1]);
         if (i & 1) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -186,13 +181,13 @@ struct Operand {
     {
         bool t = false;
 #pragma unroll
-        for (int g = 0; g < G; ++g) t |= is_tiny(big[g]);
+        for (int g = 0; g < G; ++g) t |= split_tiny(bits[g]);
         return t;
     }
-    __device__ __forceinline__ void row_max(unsigned *m, int tid) const
+    __device__ __forceinline__ void row_bits(unsigned *m, int tid) const
     {
 #pragma unroll
-        for (int g = 0; g < G; ++g) atomicMax(&m[row_of(tid, g)], __builtin_bit_cast(unsigned, big[g]));
+        for (int g = 0; g < G; ++g) atomicOr(&m[row_of(tid, g)], bits[g]);
     }
 };
 
@@ -396,18 +391,18 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
         if (oa.tiny() || ob.tiny()) tiny_row = 1;
         __syncthreads();
         if (tiny_row) {
-            // A thread saw only its share of a row's k: take the row's maximum.
+            // A thread saw only its share of a row's k: take the row's whole.
             unsigned *const ma = (unsigned *)As0, *const mb = (unsigned *)Bs0;
             for (int i = tid; i < TM; i += NT) ma[i] = 0;
             for (int i = tid; i < TN; i += NT) mb[i] = 0;
             __syncthreads();
-            oa.row_max(ma, tid);
-            ob.row_max(mb, tid);
+            oa.row_bits(ma, tid);
+            ob.row_bits(mb, tid);
             if (tid == 0) tiny_row = 0;
             __syncthreads();
             bool tiny = false;
-            for (int i = tid; i < TM; i += NT) tiny |= is_tiny(__builtin_bit_cast(float, ma[i]));
-            for (int i = tid; i < TN; i += NT) tiny |= is_tiny(__builtin_bit_cast(float, mb[i]));
+            for (int i = tid; i < TM; i += NT) tiny |= split_tiny(ma[i]);
+            for (int i = tid; i < TN; i += NT) tiny |= split_tiny(mb[i]);
             if (tiny) tiny_row = 1;
             __syncthreads();
         }

@@ -47,10 +47,18 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// A row whose largest magnitude is below this (and not 0) is left to the
-// fp32 instruction: 2^-100, so that a row that stays keeps lo down to 2^-34
-// of its largest element.
-constexpr float kSplitTiny = 7.8886090522101181e-31f;
+// A row whose largest magnitude is below 2^-95 (and not 0) is left to the
+// fp32 instruction, so that a row that stays keeps lo down to 2^-39 of its
+// largest element.  Kernels collect the bits of a row's elements with OR (one
+// operation per pair): the exponent fields' top three bits then tell.
+__device__ __forceinline__ bool split_tiny(unsigned bits)
+{
+    return (bits & 0x7fffffffu) != 0 && (bits & 0x70000000u) == 0;
+}
+__device__ __forceinline__ unsigned float_bits(float x)
+{
+    return __builtin_bit_cast(unsigned, x);
+}
 
 // The sign bit of row or column i: the top bit of i times 2^32 / golden ratio,
 // which alternates evenly over every stride of i.

@@ -1,0 +1,114 @@
+"""The split-bf16 forward (attn_fwd_kernel) where it can go wrong: lengths
+around its key tiles and query blocks in each launch form (4 or 8 waves, one
+block, two at once, two in turn), values that the split cannot carry, and its
+error against float64 next to the fp32 instruction's."""
+
+import numpy as np
+import pytest
+
+import gpu_helpers as G
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(q, k, v, causal):
+    """float64 O and LSE of (S, D) operands; a score of -inf is a weight of 0."""
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    S, D = q.shape
+    with np.errstate(invalid="ignore", over="ignore"):
+        s = q @ k.T * np.float64(np.float32(1 / np.sqrt(D)))
+    if causal:
+        s[np.triu(np.ones((S, S), bool), 1)] = -np.inf
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - m)
+    tot = p.sum(-1, keepdims=True)
+    return p @ v / tot, (m + np.log(tot))[:, 0]
+
+
+def _qkv(H, S, D, seed):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal((1, H, S, D), dtype=np.float32) for _ in range(3)]
+
+
+def _check(q, k, v, causal, heads, log=None):
+    o, lse = G.attention_fwd(q, k, v, causal, log=log)
+    for h in heads:
+        ro, rl = _ref(q[0, h], k[0, h], v[0, h], causal)
+        np.testing.assert_allclose(o[0, h], ro, rtol=1e-3, atol=2e-4)
+        np.testing.assert_allclose(lse[0, h], rl, rtol=1e-3, atol=2e-4)
+    return o, lse
+
+
+@pytest.mark.parametrize("H,S,D,causal", [
+    # 4 waves, one block: one key past a tile, one short of it, one past a block
+    (70, 129, 32, False), (70, 191, 32, True), (70, 129, 64, False), (66, 257, 64, False),
+    (70, 159, 128, False), (66, 161, 128, True), (65, 255, 128, False),
+    # 8 waves, one block
+    (300, 129, 128, False), (260, 257, 64, False), (300, 385, 32, True), (130, 511, 128, False),
+    # two blocks at once: even and odd counts, a last block of one row
+    (40, 513, 64, True), (64, 641, 128, True), (30, 385, 32, True), (65, 960, 64, True),
+    # two blocks in turn
+    (256, 512, 64, True), (256, 400, 128, True),
+])
+def test_lengths_and_launch_forms(H, S, D, causal):
+    q, k, v = _qkv(H, S, D, H + S + D)
+    log = []
+    _check(q, k, v, causal, (0, H // 2, H - 1), log)
+    assert log[0].startswith("attn_fwd_kernel"), log
+
+
+FORMS = [(70, 200, 64, False), (70, 200, 128, True), (300, 300, 128, True), (40, 640, 64, True)]
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+def test_infinite_keys_get_no_weight(H, S, D, causal):
+    """K holding -inf (times positive q) gives scores of -inf: weight 0."""
+    q, k, v = _qkv(H, S, D, 1)
+    q[..., 0] = np.abs(q[..., 0]) + 0.1
+    k[0, 3, 40:50, 0] = -np.inf
+    k[0, H - 1, S - 1, 0] = -np.inf
+    _check(q, k, v, causal, (0, 3, H - 1))
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+def test_infinite_values(H, S, D, causal):
+    """An infinite V element makes its column infinite for the rows that see
+    it and changes nothing else."""
+    q, k, v = _qkv(H, S, D, 2)
+    v[0, 9, 33, 4] = np.inf
+    o, _ = G.attention_fwd(q, k, v, causal)
+    finite = np.where(np.isinf(v[0, 9]), 0, v[0, 9])
+    ro, _ = _ref(q[0, 9], k[0, 9], finite, causal)
+    sees = np.arange(S) >= (33 if causal else 0)
+    # Masked keys of the same 32-key tile: 0 * inf is NaN, as with the fp32 instruction.
+    far = np.arange(S) < 32 if causal else np.zeros(S, bool)
+    assert np.isposinf(o[0, 9, sees, 4]).all()
+    cols = np.arange(D) != 4
+    np.testing.assert_allclose(o[0, 9][:, cols], ro[:, cols], rtol=1e-3, atol=2e-4)
+    np.testing.assert_allclose(o[0, 9, far, 4], ro[far, 4], rtol=1e-3, atol=2e-4)
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("exponent", [-100, -120])
+def test_tiny_values_keep_their_precision(H, S, D, causal, exponent):
+    """V below what three bf16 parts can hold: O to fp32 precision relative
+    to V's size."""
+    q, k, v = _qkv(H, S, D, 3)
+    v *= np.float32(2.0 ** exponent)
+    o, _ = G.attention_fwd(q, k, v, causal)
+    for h in (0, H - 1):
+        ro, _ = _ref(q[0, h], k[0, h], v[0, h], causal)
+        np.testing.assert_allclose(o[0, h] * 2.0 ** -exponent, ro * 2.0 ** -exponent, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("H,S,D,causal,o_err,lse_err", [
+    (80, 2048, 64, True, 4.2e-7, 5.9e-8), (130, 1024, 128, True, 4.0e-7, 5.6e-8), (30, 777, 128, False, 6.8e-7, 5.4e-8),
+    (130, 600, 32, False, 5.5e-7, 5.6e-8)])
+def test_error_no_larger_than_the_fp32_instructions(H, S, D, causal, o_err, lse_err):
+    """Relative 2-norm error against float64 below what the kernel on the
+    fp32 matrix instruction measured (its O errors, rounded up)."""
+    q, k, v = _qkv(H, S, D, 4)
+    o, lse = G.attention_fwd(q, k, v, causal)
+    ro, rl = zip(*(_ref(q[0, h], k[0, h], v[0, h], causal) for h in (0, 1)))
+    assert np.linalg.norm(o[0, :2] - np.stack(ro)) / np.linalg.norm(ro) <= o_err
+    assert np.linalg.norm(lse[0, :2] - np.stack(rl)) / np.linalg.norm(rl) <= lse_err
