@@ -37,7 +37,7 @@ HIP_SOURCES = [
     ("attention_fwd.hip", []),
     ("attention_fwd_tiles.hip", []),
     ("attention_bwd.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
-    ("attention_bwd_c128.hip", []),
+    ("attention_bwd_tiles.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     ("attention_bwd_s128.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     ("attention_bwd_w16.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     ("optim.hip", []),

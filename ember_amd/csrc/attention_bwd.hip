@@ -1,21 +1,17 @@
 // attention_bwd.hip -- entry point of the fused flash-attention backward
 // (fp32, gfx950); the short-sequence kernels (S <= 64: one workgroup per head
 // with Q, K, V, dO staged in LDS) are below; 64 < S <= 128 at D = 64 and 128
-// runs attn_bwd_s128 (attention_bwd_s128.hip), longer D = 64 attn_bwd_w16
-// (attention_bwd_w16.hip), and the rest the key-block workgroup kernel of
-// attention_bwd_kernels.h.
+// runs attn_bwd_s128 (attention_bwd_s128.hip), and longer ones the key-block
+// kernel on split bf16 (attention_bwd_tiles.hip) or, at D = 64 in short or
+// small launches, attn_bwd_w16 (attention_bwd_w16.hip).
 //
 // No reference counterpart (pawel002/ember has no attention): the operator is
 // new, slotted beside matmul in src/tensor/operators.h:20-27.  Its semantics
 // are those of oracle/ember_oracle.c (oracle_attention_bwd).
 //
 // Build note.  This file is compiled with -mllvm -amdgpu-mfma-vgpr-form=1
-// (MFMA accumulators in VGPRs); the causal D = 128 instantiation lives in
-// attention_bwd_c128.hip, compiled with the default (AGPR) form.  Measured
-// at config shapes on MI355X: the AGPR form is 1.7 % faster for causal
-// D = 128, while for non-causal D = 128 the default allocation cycles the
-// 128 dK/dV accumulators between AGPRs and VGPRs every query block and runs
-// 2x slower than the VGPR form (and D = 64 causal is 6 % faster in VGPR form).
+// (MFMA accumulators in VGPRs): the default allocation cycles accumulators
+// that vector instructions read between AGPRs and VGPRs.
 #include <mutex>
 
 #include <algorithm>
@@ -801,6 +797,18 @@ int attention_bwd_rows(const float *q, const float *k, const float *v, const flo
     args.order = order;
     args.order_timeouts = timeouts;
     args.order_group = 1;
+    // D = 64: 16-key chunks, four workgroups of 64 keys per CU
+    // (attention_bwd_w16.hip), for walks of up to 512 queries, which do not
+    // cover the longer prologue of the key-block kernel (128 keys, one
+    // workgroup per CU: 128 heads of 200 causal 41 against 38 us, 512 of 130
+    // 110 against 85, 32 of 512 69 against 65; 128 causal of 512 102 against
+    // 120) and for launches of fewer than 64 key blocks, where neither fills
+    // the chip (6 heads of 1024 causal, 48 blocks, 116 against 135; 16 heads,
+    // 128 blocks, 119 against 137).  Beyond: 30 heads of 777 107 against 147
+    // us, 32 of 1024 141 against 191, 128 of 2048 causal 1159 against 1389.
+    // The rule does not look at deterministic(): dK and dV are the same bits
+    // in both modes.
+    const bool w16 = D == 64 && (S <= 512 || nkb * B * H < 64);
     if (ordered && causal) {
         // Key blocks per group of the dQ order (attention_bwd_kernels.h): as
         // many as run at once per head, R = slots / heads (B * H rounded up
@@ -809,7 +817,7 @@ int attention_bwd_rows(const float *q, const float *k, const float *v, const flo
         // Non-causal walks all start at the first tile, where no key block
         // is ahead of another: R = 1 (ascending).
         const int ncu = device_cu_count();
-        const int per_cu = D == 64 ? 4 : D == 32 ? 2 : 1;  // workgroups per CU (LDS, registers)
+        const int per_cu = w16 ? 4 : D == 32 ? 2 : 1;  // workgroups per CU (LDS, registers)
         const int64_t slots = (int64_t)ncu * per_cu;
         const int64_t heads8 = (B * H + 7) / 8 * 8;
         int64_t R = std::min<int64_t>(nkb, slots / heads8);
@@ -829,15 +837,8 @@ int attention_bwd_rows(const float *q, const float *k, const float *v, const flo
     args.out_sh = out_sh;
     args.out_ss = out_ss;
     const int nblocks = args.nkb * (int)(B * H);
-    // D = 64: 16-key chunks, four workgroups per CU (attention_bwd_w16.hip);
-    // D = 32 and 128: the key-block workgroup kernel.
-    if (D == 64) return launch_bwd_w16(args, rows_pad, causal != 0, (int)(B * H));
-    switch (D * 2 + (causal ? 1 : 0)) {
-        case 64: return launch_bwd<32, false>(args, rows_pad, nblocks);
-        case 65: return launch_bwd<32, true>(args, rows_pad, nblocks);
-        case 256: return launch_bwd<128, false>(args, rows_pad, nblocks);
-        default: return launch_bwd_causal_d128(args, rows_pad, nblocks);
-    }
+    if (w16) return launch_bwd_w16(args, rows_pad, causal != 0, (int)(B * H));
+    return launch_bwd_tiles(args, (int)D, causal != 0, rows_pad, nblocks);
 }
 
 }  // namespace

@@ -5,11 +5,11 @@
 // those of oracle/ember_oracle.c (oracle_attention_bwd).
 //
 // Why a kernel of its own.  The key-block workgroup kernel
-// (attention_bwd_kernels.h) gives each of its 4 waves 32 keys and walks
+// (attention_bwd_tiles.hip) gives each of its 4 waves 32 keys and walks
 // 32-query blocks in lockstep; at S = 128 that is one workgroup per head in
 // which, causally, wave 0 has work in all 4 steps and wave 3 in one, so a
 // causal head costs as much as a non-causal one (measured 1.98 against
-// 2.00 ms at B128 H64 D128).  Here the keys are cut into 16-row chunks and
+// 2.00 ms at B128 H64 D128, its products then on the fp32 instruction).  Here the keys are cut into 16-row chunks and
 // every product runs on v_mfma_f32_16x16x4f32, so that masked work is cut at
 // 16 x 16 and the chunks can be dealt out evenly: a causal chunk j is seen
 // by 8 - j of the 8 query chunks, and the chunks j and 7 - j together by 9,

@@ -1,23 +1,20 @@
-// attention_bwd_w16.hip -- the fused attention backward for S > 128 at
-// head_dim 64, in 16-key chunks (attn_bwd_w16).
+// attention_bwd_w16.hip -- the fused attention backward at head_dim 64 for
+// 128 < S <= 512 and for small launches, in 16-key chunks (attn_bwd_w16) on
+// the fp32 matrix instruction.
 //
 // No reference counterpart (pawel002/ember has no attention); semantics are
 // those of oracle/ember_oracle.c (oracle_attention_bwd).
 //
-// The key-block kernel (attention_bwd_kernels.h) gives each of its 4 waves 32
-// keys on v_mfma_f32_32x32x2f32 and walks 32-query blocks; at D = 64 it takes
-// 272 registers per lane and 104 KB of LDS, so a CU runs one workgroup, one
-// wave per SIMD, every wait in a step (barriers, LDS latency, the atomics'
-// issue) idles the matrix core, and causally each workgroup computes 128 x
-// 128 diagonal scores of which half are masked.  Here a workgroup holds 64
-// keys, one 16-key chunk per wave on v_mfma_f32_16x16x4f32 (the same rate per
-// flop): K, V, dK, dV of a chunk take 4 x 16 registers per lane (126 in
-// all), and the LDS holds two 16-query chunk sets, the dS of one chunk and
-// K^T of the 64 keys (39 KB), so four independent workgroups share a CU and
-// fill each other's waits, and masked work is cut at 16 x 16.  (Three per CU
-// with a second dS buffer and one barrier per step measured 3-6 % slower.)  At D = 128 the same design
-// (188 registers, 79 KB, two workgroups per CU) measured 5-7 % slower than
-// the key-block kernel, which keeps that case.
+// The key-block kernel (attention_bwd_tiles.hip) has the faster products, but
+// one workgroup of 128 keys fills a CU's LDS, and splitting K and V before its
+// first product takes as long as several steps.  Here a workgroup holds 64
+// keys, one 16-key chunk per wave on v_mfma_f32_16x16x4f32: K, V, dK, dV of a
+// chunk take 4 x 16 registers per lane (126 in all), and the LDS holds two
+// 16-query chunk sets, the dS of one chunk and K^T of the 64 keys (39 KB), so
+// four independent workgroups share a CU and fill each other's waits, and
+// masked work is cut at 16 x 16.  (Three per CU with a second dS buffer and
+// one barrier per step measured 3-6 % slower.)  Measured on both sides at the
+// rule that chooses (attention_bwd.hip).
 //
 // Per step qc (16 query rows), as attn_bwd_s128:
 //   dQ of chunk qc - 2 (formed in the previous step) added into dq;
@@ -364,10 +361,9 @@ int launch_w16(const BwdArgs &args, int64_t rows_pad, int nbh)
     const dim3 grid((unsigned)(nkb * nbh));
     if (!args.order) {
         // Causal launches whose key-block pairs all fit one round of resident
-        // workgroups take the blocks in pairs of about equal walks: measured
-        // +4 % at B4 H16 S = 1024, +8-9 % at B2 H16 S = 2048 and B1 H16
-        // S = 4096, +-0 at B8 H16 S = 1024; at S = 512 (short walks, which do
-        // not cover the second block's prologue) -2.5 %, so from 16 blocks.
+        // workgroups take the blocks in pairs of about equal walks, from 16
+        // blocks (measured at 64 heads of 1024 +4 %, 32 of 2048 +8-9 %; at S =
+        // 512 short walks do not cover the second block's prologue, -2.5 %).
         if constexpr (CAUSAL) {
             const int ncu = device_cu_count();
             const int64_t pairs = (int64_t)(nkb + 1) / 2 * nbh;

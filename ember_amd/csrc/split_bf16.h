@@ -90,6 +90,20 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsi
     l = pack_bf16(x0, x1);
 }
 
+// The same for values up to the largest fp32 number, which bf16 would round up
+// to infinity.
+__device__ __forceinline__ void split_pair_full(float x0, float x1, unsigned &h, unsigned &m, unsigned &l)
+{
+    const float top = __builtin_bit_cast(float, 0x7f7f0000u);
+    h = pack_bf16(__builtin_amdgcn_fmed3f(x0, -top, top), __builtin_amdgcn_fmed3f(x1, -top, top));
+    x0 -= __builtin_bit_cast(float, h << 16);
+    x1 -= __builtin_bit_cast(float, h & 0xffff0000u);
+    m = pack_bf16(x0, x1);
+    x0 -= __builtin_bit_cast(float, m << 16);
+    x1 -= __builtin_bit_cast(float, m & 0xffff0000u);
+    l = pack_bf16(x0, x1);
+}
+
 // Eight floats as the three parts of one operand.
 struct Split8 {
     u32x4 part[3];  // hi, mid, lo
