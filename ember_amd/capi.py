@@ -79,6 +79,8 @@ def lib() -> C.CDLL:
     L.attention_bwd_noalloc.argtypes = [_vp] * 9 + [_i64] * 4 + [C.c_float, C.c_int] + [_i64] * 6
     L.softmax_axis.restype = C.c_int
     L.softmax_axis.argtypes = [_vp, _vp, C.c_int, C.c_int, C.c_int]
+    L.cross_entropy_loss.restype = C.c_int
+    L.cross_entropy_loss.argtypes = [_vp] * 4 + [C.c_int, C.c_int, C.c_float, C.POINTER(C.c_float)]
     L.gemm_ex.restype = C.c_int
     L.gemm_ex.argtypes = [_vp] * 3 + [C.c_int] * 6 + [_vp] * 3 + [C.c_int]
     L.ember_set_deterministic.argtypes = [C.c_int]

@@ -27,6 +27,9 @@ bool launch_ok(const char *kernel);
 // the caller can do without, so that running out of memory gives null but
 // records no error.
 void *scratch(int slot, size_t bytes, bool optional = false);
+// The sum of n device doubles as one host float, through device memory `res`;
+// synchronises (elementwise.hip).
+int sum_partials(const double *partial, int n, float *res, float *host, const char *who);
 
 enum ScratchSlot {
     kScratchAttnDelta = 0,

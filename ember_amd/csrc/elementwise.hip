@@ -366,6 +366,19 @@ __global__ __launch_bounds__(64) void k_reduce_rows_ring(const float *a, float *
 
 }  // namespace
 
+namespace ember {
+
+// The sum of n doubles in a fixed tree order, as one float on the host (res:
+// device memory for it).
+int sum_partials(const double *partial, int n, float *res, float *host, const char *who)
+{
+    hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, 0, partial, n, res);
+    if (!launch_ok(who)) return EMBER_ERR_DEVICE;
+    return hip_ok(hipMemcpy(host, res, sizeof(float), hipMemcpyDeviceToHost), who) ? EMBER_OK : EMBER_ERR_DEVICE;
+}
+
+}  // namespace ember
+
 extern "C" {
 
 void transpose(const float *a, float *out, int n, int m)
@@ -385,10 +398,8 @@ float sum(const float *a, int size)
     double *partial = (double *)ws;
     float *res = (float *)(ws + (size_t)nblk * sizeof(double));
     hipLaunchKernelGGL(k_sum_partial, dim3(nblk), dim3(kBlock), 0, 0, a, size, partial);
-    hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, 0, partial, nblk, res);
-    if (!ember::launch_ok("sum")) return 0.0f;
     float host = 0.0f;
-    ember::hip_ok(hipMemcpy(&host, res, sizeof(float), hipMemcpyDeviceToHost), "sum");
+    ember::sum_partials(partial, nblk, res, &host, "sum");
     return host;
 }
 
@@ -404,11 +415,7 @@ int mse_loss(const float *pred, const float *target, float *grad, int size, floa
     double *partial = (double *)ws;
     float *res = (float *)(ws + (size_t)nblk * sizeof(double));
     hipLaunchKernelGGL(k_mse_partial, dim3(nblk), dim3(kBlock), 0, 0, pred, target, grad, scale, size, partial);
-    hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, 0, partial, nblk, res);
-    if (!ember::launch_ok("mse_loss")) return EMBER_ERR_DEVICE;
-    if (!ember::hip_ok(hipMemcpy(loss, res, sizeof(float), hipMemcpyDeviceToHost), "mse_loss"))
-        return EMBER_ERR_DEVICE;
-    return EMBER_OK;
+    return ember::sum_partials(partial, nblk, res, loss, "mse_loss");
 }
 
 int sum_axis_product(const int *shape, int start, int end)

@@ -1,4 +1,5 @@
-// softmax.hip -- softmax along one axis in one launch.
+// softmax.hip -- softmax along one axis in one launch, and the softmax
+// cross-entropy loss (below).
 //
 // Ember's softmax(a, axis) is exp(a - amax(a, axis)) / sum(exp(...), axis)
 // (ember/tensor/tensor.py:430-437), run by the reference as five launches
@@ -19,6 +20,8 @@
 //     coalesced across inner.
 // HBM-bound: 8 bytes per element (read + write) on the first two paths.
 #include <math.h>
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -165,6 +168,150 @@ void launch_wave(const float *a, float *out, int rows, int L)
     hipLaunchKernelGGL(softmax_rows_wave<NV>, dim3((rows + 3) / 4), dim3(256), 0, 0, a, out, rows, L);
 }
 
+// ---- softmax cross-entropy ----
+// Ember's CrossEntropyLoss (ember/loss/losses.py:29-56) composes nine
+// element-wise, reduction and broadcast launches, each a pass over the logits'
+// size; one pass here.  Per row: m = max, s = sum of expf(x - m), logp = (x -
+// m) - logf(s), p = expf(logp), grad = (p - t) / n, and the sum of t * logp,
+// in the composition's fp32 operations except for the order of s; the
+// products are summed in double, per workgroup.
+//
+// HBM-bound: 16 bytes per element, two arrays read and two written.  A row is
+// held in the registers of 16, 32 or 64 lanes (16 floats per lane at 1000
+// classes), logits and targets loaded together; rows longer than 4096 (1024
+// where they are not 16-byte aligned, one float per load) take a workgroup
+// each and three passes, of which the second and third hit the caches.
+// Value and gradient of 8192 x 1000 with the sum read back: composed 179 us, 50
+// here; 64 x 10 in the training step of a small classifier: step 114 -> 87 us.
+constexpr int kLossBlocks = 2048;  // 8 workgroups of 4 waves per CU
+
+template <int TPR>
+__device__ __forceinline__ float group_max(float v)
+{
+#pragma unroll
+    for (int o = TPR / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+template <int TPR>
+__device__ __forceinline__ float group_sum(float v)
+{
+#pragma unroll
+    for (int o = TPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+struct LossArgs {
+    const float *x, *t;
+    float *probs, *grad;
+    double *partial;  // one per workgroup
+    int rows, L;
+    float n;
+};
+
+// The element's outputs; returns t * logp, rounded as the composition's product.
+__device__ __forceinline__ float loss_element(float shifted, float logs, float t, float n, float &p, float &g)
+{
+#pragma clang fp contract(off)
+    const float logp = shifted - logs;
+    p = expf(logp);
+    g = (p - t) / n;
+    return t * logp;
+}
+
+__device__ __forceinline__ void store_partial(double sum, double *partial)
+{
+    __shared__ double red[4];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// TPR lanes per row, NV pieces of W neighbouring floats per lane (TPR * NV * W >= L).
+template <int TPR, int NV, int W>
+__global__ __launch_bounds__(256) void cross_entropy_rows(LossArgs a)
+{
+    typedef float piece __attribute__((ext_vector_type(W)));
+    constexpr int RPB = 256 / TPR;
+    const int sub = threadIdx.x % TPR;
+    double sum = 0.0;
+    for (int row = blockIdx.x * RPB + threadIdx.x / TPR; row < a.rows; row += gridDim.x * RPB) {
+        const int64_t base = (int64_t)row * a.L;
+        piece x[NV], t[NV];
+        float m = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = W * (TPR * j + sub);
+            if (c < a.L) {
+                x[j] = *(const piece *)(a.x + base + c);
+                t[j] = *(const piece *)(a.t + base + c);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            if (W * (TPR * j + sub) < a.L)
+#pragma unroll
+                for (int e = 0; e < W; ++e) m = fmaxf(m, x[j][e]);
+        m = group_max<TPR>(m);
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            if (W * (TPR * j + sub) < a.L)
+#pragma unroll
+                for (int e = 0; e < W; ++e) {
+                    x[j][e] -= m;
+                    s += expf(x[j][e]);
+                }
+        const float logs = logf(group_sum<TPR>(s));
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = W * (TPR * j + sub);
+            if (c < a.L) {
+                piece p, g;
+#pragma unroll
+                for (int e = 0; e < W; ++e) {
+                    float pe, ge;
+                    sum += (double)loss_element(x[j][e], logs, t[j][e], a.n, pe, ge);
+                    p[e] = pe, g[e] = ge;
+                }
+                *(piece *)(a.probs + base + c) = p;
+                *(piece *)(a.grad + base + c) = g;
+            }
+        }
+    }
+    store_partial(sum, a.partial);
+}
+
+__global__ __launch_bounds__(256) void cross_entropy_long(LossArgs a)
+{
+    __shared__ float red[4];
+    double sum = 0.0;
+    for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
+        const int64_t base = (int64_t)row * a.L;
+        const float *x = a.x + base, *t = a.t + base;
+        float m = -INFINITY, s = 0.0f;
+        for (int c = threadIdx.x; c < a.L; c += 256) m = fmaxf(m, x[c]);
+        m = block_reduce<true>(m, red);
+        for (int c = threadIdx.x; c < a.L; c += 256) s += expf(x[c] - m);
+        const float logs = logf(block_reduce<false>(s, red));
+        for (int c = threadIdx.x; c < a.L; c += 256) {
+            float p, g;
+            sum += (double)loss_element(x[c] - m, logs, t[c], a.n, p, g);
+            a.probs[base + c] = p;
+            a.grad[base + c] = g;
+        }
+    }
+    store_partial(sum, a.partial);
+}
+
+template <int TPR, int NV, int W>
+void launch_loss(const LossArgs &a, int blocks)
+{
+    hipLaunchKernelGGL((cross_entropy_rows<TPR, NV, W>), dim3(blocks), dim3(256), 0, 0, a);
+}
+
 }  // namespace
 }  // namespace ember
 
@@ -194,4 +341,42 @@ extern "C" int softmax_axis(const float *a, float *out, int outer, int inner, in
                            inner, axis_dim);
     }
     return launch_ok("softmax_axis") ? EMBER_OK : EMBER_ERR_DEVICE;
+}
+
+extern "C" int cross_entropy_loss(const float *logits, const float *target, float *probs, float *grad, int rows,
+                                  int classes, float n, float *total)
+{
+    using namespace ember;
+    if (rows < 0 || classes < 0 || !total) return record_error(EMBER_ERR_INVALID_ARGUMENT, "cross_entropy_loss");
+    *total = 0.0f;
+    if (rows == 0 || classes == 0) return EMBER_OK;
+    if (!logits || !target || !probs || !grad) return record_error(EMBER_ERR_INVALID_ARGUMENT, "cross_entropy_loss");
+    const int L = classes;
+    const bool quads = L % 4 == 0 &&
+                       (((uintptr_t)logits | (uintptr_t)target | (uintptr_t)probs | (uintptr_t)grad) & 15) == 0;
+    const bool by_block = L > (quads ? 4096 : 1024);
+    const int per_block = by_block ? 1 : L <= 16 ? 16 : L <= 32 ? 8 : 4;  // rows
+    const int blocks = (int)std::min<int64_t>(((int64_t)rows + per_block - 1) / per_block, kLossBlocks);
+    char *ws = (char *)scratch(kScratchSum, (size_t)blocks * sizeof(double) + 16);
+    if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
+    const LossArgs a = {logits, target, probs, grad, (double *)ws, rows, L, n};
+    if (L <= 16) launch_loss<16, 1, 1>(a, blocks);
+    else if (L <= 32) launch_loss<32, 1, 1>(a, blocks);
+    else if (by_block) hipLaunchKernelGGL(cross_entropy_long, dim3(blocks), dim3(256), 0, 0, a);
+    else if (quads) {
+        if (L <= 256) launch_loss<64, 1, 4>(a, blocks);
+        else if (L <= 512) launch_loss<64, 2, 4>(a, blocks);
+        else if (L <= 1024) launch_loss<64, 4, 4>(a, blocks);
+        else if (L <= 2048) launch_loss<64, 8, 4>(a, blocks);
+        else launch_loss<64, 16, 4>(a, blocks);
+    } else {
+        if (L <= 64) launch_loss<64, 1, 1>(a, blocks);
+        else if (L <= 128) launch_loss<64, 2, 1>(a, blocks);
+        else if (L <= 256) launch_loss<64, 4, 1>(a, blocks);
+        else if (L <= 512) launch_loss<64, 8, 1>(a, blocks);
+        else launch_loss<64, 16, 1>(a, blocks);
+    }
+    if (!launch_ok("cross_entropy_loss")) return EMBER_ERR_DEVICE;
+    return sum_partials((double *)ws, blocks, (float *)(ws + (size_t)blocks * sizeof(double)), total,
+                        "cross_entropy_loss");
 }

@@ -521,6 +521,36 @@ static PyObject *py_mse_loss(PyObject *module, PyObject *args)
     return Py_BuildValue("(dN)", (double)loss, (PyObject *)g);
 }
 
+/* _cross_entropy_loss(logits, target, rows, n) -> (sum of target * log_softmax,
+ * probs, grad): one pass for CrossEntropyLoss (see cross_entropy_loss). */
+static PyObject *py_cross_entropy_loss(PyObject *module, PyObject *args)
+{
+    TensorObject *x, *t;
+    Py_ssize_t rows;
+    float n;
+    (void)module;
+    if (!PyArg_ParseTuple(args, "O!O!nf", &TensorType, &x, &TensorType, &t, &rows, &n)) return NULL;
+    if (x->size != t->size || rows <= 0 || x->size % rows) {
+        PyErr_SetString(PyExc_ValueError, "_cross_entropy_loss: size mismatch");
+        return NULL;
+    }
+    if (!fits_int(x->size, "_cross_entropy_loss")) return NULL;
+    TensorObject *p = alloc_tensor(x->size);
+    TensorObject *g = p ? alloc_tensor(x->size) : NULL;
+    if (!g) {
+        Py_XDECREF(p);
+        return NULL;
+    }
+    float total = 0.0f;
+    int st = cross_entropy_loss(x->d_ptr, t->d_ptr, p->d_ptr, g->d_ptr, (int)rows, (int)(x->size / rows), n, &total);
+    if (raise_status(st, "_cross_entropy_loss")) {
+        Py_DECREF(p);
+        Py_DECREF(g);
+        return NULL;
+    }
+    return Py_BuildValue("(dNN)", (double)total, (PyObject *)p, (PyObject *)g);
+}
+
 typedef void (*axis_fn)(const float *, float *, int, int, int);
 
 static PyObject *do_axis(PyObject *args, axis_fn fn, const char *what)
@@ -1107,6 +1137,7 @@ static PyMethodDef module_methods[] = {
     METHOD("_from_numpy", py_from_numpy, "float32 C-contiguous buffer -> _Tensor"),
     METHOD("_sum", py_sum, "sum of all elements"),
     METHOD("_mse_loss", py_mse_loss, "MSE loss sum and gradient in one pass"),
+    METHOD("_cross_entropy_loss", py_cross_entropy_loss, "softmax cross-entropy sum, probabilities and gradient in one pass"),
     METHOD("_sum_axis", py_sum_axis, "sum over one axis"),
     METHOD("_max_axis", py_max_axis, "max over one axis"),
     METHOD("_softmax", py_softmax, "softmax along one axis, one launch"),

@@ -59,16 +59,27 @@ class CrossEntropyLoss(Loss):
     """Softmax cross-entropy over (batch, classes) logits against one-hot (or
     probability) targets, averaged over the batch (``losses.py:29-56``):
     forward -sum(target * log_softmax(pred)) / batch with the log-sum-exp
-    shift; backward (softmax(pred) - target) / batch."""
+    shift; backward (softmax(pred) - target) / batch.
+
+    Equal shapes take one fused pass (``_cross_entropy_loss``) that forms the
+    gradient with the probabilities; broadcasting shapes compose the operators
+    as the reference."""
 
     def __init__(self) -> None:
         self.probs: Tensor | None = None
         self.target: Tensor | None = None
+        self.grad: Tensor | None = None
         self.n = 0
 
     def forward(self, pred: Tensor, target: Tensor) -> float:
         self.n = pred.shape[0]
         self.target = target
+        self.grad = None
+        if isinstance(pred, Tensor) and isinstance(target, Tensor) and pred.shape == target.shape and math.prod(pred.shape):
+            rows = math.prod(pred.shape[:-1])
+            total, p, g = C._cross_entropy_loss(pred._core, target._core, rows, self.n)
+            self.probs, self.grad = Tensor._from_core(p, pred.shape), Tensor._from_core(g, pred.shape)
+            return -total / self.n
         shifted = pred - amax(pred, axis=-1, keepdims=True)
         log_probs = shifted - log(_sum(exp(shifted), axis=-1, keepdims=True))
         self.probs = exp(log_probs)
@@ -77,6 +88,8 @@ class CrossEntropyLoss(Loss):
     def backward(self) -> Tensor:
         if self.probs is None or self.target is None:
             raise RuntimeError("forward() must run before backward()")
+        if self.grad is not None:
+            return self.grad
         return (self.probs - self.target) / self.n
 
 

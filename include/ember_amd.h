@@ -145,6 +145,13 @@ float sum(const float *a, int size);
  * No reference counterpart as one symbol: it fuses sub_tensor, mul_tensor,
  * sum and mul_scalar.  Synchronises (the loss is read back). */
 int mse_loss(const float *pred, const float *target, float *grad, int size, float scale, float *loss);
+/* Ember's CrossEntropyLoss over (rows, classes) in one pass
+ * (ember/loss/losses.py:29-56): probs = softmax(logits), grad = (probs -
+ * target) / n, *total = sum of target * log_softmax(logits), in the fp32
+ * operations of the composed operators but for the order of a row's sum.  No
+ * reference counterpart as one symbol.  Synchronises (the sum is read back). */
+int cross_entropy_loss(const float *logits, const float *target, float *probs, float *grad, int rows, int classes,
+                       float n, float *total);
 /* Product of shape[start:end]; replaces operators_gpu.cu:168-173. */
 int sum_axis_product(const int *shape, int start, int end);
 /* Reduce the middle axis of (outer, axis_dim, inner); sequential fp32 sum /
