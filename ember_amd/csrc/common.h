@@ -27,9 +27,10 @@ bool launch_ok(const char *kernel);
 // the caller can do without, so that running out of memory gives null but
 // records no error.
 void *scratch(int slot, size_t bytes, bool optional = false);
-// The sum of n device doubles as one host float, through device memory `res`;
-// synchronises (elementwise.hip).
-int sum_partials(const double *partial, int n, float *res, float *host, const char *who);
+// Eight bytes of pinned host memory that every device can write, or null where
+// none are free; for the caller alone until released.
+uint64_t *host_slot();
+void release_host_slot(uint64_t *slot);
 
 enum ScratchSlot {
     kScratchAttnDelta = 0,

@@ -10,7 +10,7 @@
 //    (operators_gpu.cu:94-106);
 //  * transpose goes through a 32 x 33 LDS tile so loads and stores are both
 //    coalesced (operators_gpu.cu:138-151 stores with a stride of n);
-//  * sum() reduces on the device in double and copies one float back,
+//  * sum() reduces on the device in double and writes one float to the host,
 //    instead of copying the whole tensor to the host (operators_gpu.cu:153-166).
 // sum_axis / max_axis keep the reference's arithmetic exactly: each output is
 // folded along the axis in index order with a float accumulator (sum from
@@ -21,6 +21,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "host_sum.h"
 #include "lds_dma.h"
 #include "mfma.h"
 
@@ -161,7 +162,7 @@ __global__ void k_transpose(const float *a, float *out, int n, int m)
     }
 }
 
-__global__ void k_sum_partial(const float *a, int size, double *partial)
+__global__ void k_sum(const float *a, int size, double *partial, uint64_t *out)
 {
     __shared__ double red[kBlock];
     double s = 0.0;
@@ -173,15 +174,15 @@ __global__ void k_sum_partial(const float *a, int size, double *partial)
         if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+    ember::finish_sum(red[0], partial, out);
 }
 
-// The MSE loss in one pass: d = p - t; grad = d * scale; partial sums of
-// d*d exactly as k_sum_partial forms them over the product tensor (same
+// The MSE loss in one pass: d = p - t; grad = d * scale; the sum of
+// d*d exactly as k_sum forms them over the product tensor (same
 // grid, same strided walk, same tree), so the loss equals
 // sum(diff * diff) and grad equals scale * diff bit for bit.
-__global__ void k_mse_partial(const float *p, const float *t, float *grad, float scale, int size,
-                              double *partial)
+__global__ void k_mse(const float *p, const float *t, float *grad, float scale, int size, double *partial,
+                      uint64_t *out)
 {
 #pragma clang fp contract(off)
     __shared__ double red[kBlock];
@@ -198,21 +199,7 @@ __global__ void k_mse_partial(const float *p, const float *t, float *grad, float
         if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-__global__ void k_sum_final(const double *partial, int n, float *out)
-{
-    __shared__ double red[kBlock];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = (float)red[0];
+    ember::finish_sum(red[0], partial, out);
 }
 
 __global__ void k_sum_axis(const float *a, float *out, int outer, int inner, int axis_dim)
@@ -366,19 +353,6 @@ __global__ __launch_bounds__(64) void k_reduce_rows_ring(const float *a, float *
 
 }  // namespace
 
-namespace ember {
-
-// The sum of n doubles in a fixed tree order, as one float on the host (res:
-// device memory for it).
-int sum_partials(const double *partial, int n, float *res, float *host, const char *who)
-{
-    hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, 0, partial, n, res);
-    if (!launch_ok(who)) return EMBER_ERR_DEVICE;
-    return hip_ok(hipMemcpy(host, res, sizeof(float), hipMemcpyDeviceToHost), who) ? EMBER_OK : EMBER_ERR_DEVICE;
-}
-
-}  // namespace ember
-
 extern "C" {
 
 void transpose(const float *a, float *out, int n, int m)
@@ -396,10 +370,12 @@ float sum(const float *a, int size)
     char *ws = (char *)ember::scratch(ember::kScratchSum, (size_t)nblk * sizeof(double) + 16);
     if (!ws) return 0.0f;
     double *partial = (double *)ws;
-    float *res = (float *)(ws + (size_t)nblk * sizeof(double));
-    hipLaunchKernelGGL(k_sum_partial, dim3(nblk), dim3(kBlock), 0, 0, a, size, partial);
+    uint64_t *res = (uint64_t *)(ws + (size_t)nblk * sizeof(double));
+    const ember::HostSum result(res);
+    hipLaunchKernelGGL(k_sum, dim3(nblk), dim3(kBlock), 0, 0, a, size, partial, result.out());
+    if (!ember::launch_ok("sum")) return 0.0f;
     float host = 0.0f;
-    ember::sum_partials(partial, nblk, res, &host, "sum");
+    result.read(&host, "sum");
     return host;
 }
 
@@ -413,9 +389,11 @@ int mse_loss(const float *pred, const float *target, float *grad, int size, floa
     char *ws = (char *)ember::scratch(ember::kScratchSum, (size_t)nblk * sizeof(double) + 16);
     if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
     double *partial = (double *)ws;
-    float *res = (float *)(ws + (size_t)nblk * sizeof(double));
-    hipLaunchKernelGGL(k_mse_partial, dim3(nblk), dim3(kBlock), 0, 0, pred, target, grad, scale, size, partial);
-    return ember::sum_partials(partial, nblk, res, loss, "mse_loss");
+    uint64_t *res = (uint64_t *)(ws + (size_t)nblk * sizeof(double));
+    const ember::HostSum result(res);
+    hipLaunchKernelGGL(k_mse, dim3(nblk), dim3(kBlock), 0, 0, pred, target, grad, scale, size, partial,
+                       result.out());
+    return ember::launch_ok("mse_loss") ? result.read(loss, "mse_loss") : EMBER_ERR_DEVICE;
 }
 
 int sum_axis_product(const int *shape, int start, int end)

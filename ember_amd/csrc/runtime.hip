@@ -145,6 +145,39 @@ void release_scratch(int dev)
     }
 }
 
+// Pinned result slots: one page for the process's life, a cache line each.
+namespace {
+constexpr int kHostSlots = 64, kHostSlotWords = 8;
+std::mutex g_host_slot_mu;
+uint64_t *g_host_page = nullptr;
+bool g_host_page_tried = false;
+uint64_t g_host_slots_used = 0;
+}  // namespace
+
+uint64_t *host_slot()
+{
+    std::lock_guard<std::mutex> lock(g_host_slot_mu);
+    if (!g_host_page_tried) {
+        g_host_page_tried = true;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kHostSlots * kHostSlotWords * sizeof(uint64_t), hipHostMallocPortable | hipHostMallocMapped) ==
+            hipSuccess)
+            g_host_page = (uint64_t *)p;
+        else
+            (void)hipGetLastError();
+    }
+    if (!g_host_page || g_host_slots_used == ~0ull) return nullptr;
+    const int i = __builtin_ctzll(~g_host_slots_used);
+    g_host_slots_used |= 1ull << i;
+    return g_host_page + i * kHostSlotWords;
+}
+
+void release_host_slot(uint64_t *slot)
+{
+    std::lock_guard<std::mutex> lock(g_host_slot_mu);
+    g_host_slots_used &= ~(1ull << ((slot - g_host_page) / kHostSlotWords));
+}
+
 namespace {
 std::atomic<int> g_deterministic{0};
 std::atomic<int> g_cu_count[kMaxDevices];

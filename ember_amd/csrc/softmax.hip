@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "host_sum.h"
 
 namespace ember {
 namespace {
@@ -171,19 +172,25 @@ void launch_wave(const float *a, float *out, int rows, int L)
 // ---- softmax cross-entropy ----
 // Ember's CrossEntropyLoss (ember/loss/losses.py:29-56) composes nine
 // element-wise, reduction and broadcast launches, each a pass over the logits'
-// size; one pass here.  Per row: m = max, s = sum of expf(x - m), logp = (x -
-// m) - logf(s), p = expf(logp), grad = (p - t) / n, and the sum of t * logp,
-// in the composition's fp32 operations except for the order of s; the
-// products are summed in double, per workgroup.
+// size; one pass here.  Per row: m = max, e = expf(x - m), s = sum of e, p = e
+// * (1 / s) (nearer to the exact value than the composition's expf(logp),
+// whose exponent has been rounded), grad = (p - t) / n, and the sum of t * logp
+// with logp = (x - m) - logf(s), rounded as the composition's products and
+// added in double.
 //
-// HBM-bound: 16 bytes per element, two arrays read and two written.  A row is
-// held in the registers of 16, 32 or 64 lanes (16 floats per lane at 1000
-// classes), logits and targets loaded together; rows longer than 4096 (1024
-// where they are not 16-byte aligned, one float per load) take a workgroup
-// each and three passes, of which the second and third hit the caches.
-// Value and gradient of 8192 x 1000 with the sum read back: composed 179 us, 50
-// here; 64 x 10 in the training step of a small classifier: step 114 -> 87 us.
-constexpr int kLossBlocks = 2048;  // 8 workgroups of 4 waves per CU
+// HBM-bound where rows are long: 16 bytes per element, two arrays read and two
+// written.  A row is held in the registers of 16, 32 or 64 lanes (16 floats
+// per lane at 1000 classes); a wave loads its next row's logits and targets
+// before it works on the one it has, as the vector work (13 us of the 41 at
+// 8192 x 1000 without that) otherwise has no loads beside it.  Rows longer
+// than 4096 (1024 where they are not 16-byte aligned, one float per load) take
+// a workgroup each and three passes, of which the second and third hit the
+// caches.
+// Measured, value and gradient with the sum read back, composed and here: 8192
+// x 1000 179 and 37 us (the kernel 40 us without the next row's loads and with
+// a second expf and a division per element, 30 with them: 4.4 TB/s), 8192 x
+// 4096 688 and 137, 8192 x 1001 257 and 34, 64 x 10 60 and 14.
+constexpr int kLossBlocks = 1024;  // 4 workgroups of 4 waves per CU
 
 template <int TPR>
 __device__ __forceinline__ float group_max(float v)
@@ -205,28 +212,37 @@ struct LossArgs {
     const float *x, *t;
     float *probs, *grad;
     double *partial;  // one per workgroup
+    uint64_t *total;
     int rows, L;
     float n;
 };
 
-// The element's outputs; returns t * logp, rounded as the composition's product.
-__device__ __forceinline__ float loss_element(float shifted, float logs, float t, float n, float &p, float &g)
+// a / n with r = 1 / n: the quotient corrected by its exact remainder
+// (Markstein's method), and the special cases of a division.
+__device__ __forceinline__ float divide_by(float a, float n, float r)
 {
-#pragma clang fp contract(off)
-    const float logp = shifted - logs;
-    p = expf(logp);
-    g = (p - t) / n;
-    return t * logp;
+    const float q = a * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, n, a), r, q), n, a);
 }
 
-__device__ __forceinline__ void store_partial(double sum, double *partial)
+// The element's outputs; returns t * logp, rounded as the composition's product.
+__device__ __forceinline__ float loss_element(float shifted, float logs, float e, float inv, float t, float n, float r,
+                                              float &p, float &g)
 {
-    __shared__ double red[4];
+#pragma clang fp contract(off)
+    p = e * inv;
+    g = divide_by(p - t, n, r);
+    return t * (shifted - logs);
+}
+
+__device__ __forceinline__ void store_sum(double sum, const LossArgs &a)
+{
+    __shared__ double waves[4];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    finish_sum((waves[0] + waves[1]) + (waves[2] + waves[3]), a.partial, a.total);
 }
 
 // TPR lanes per row, NV pieces of W neighbouring floats per lane (TPR * NV * W >= L).
@@ -236,57 +252,72 @@ __global__ __launch_bounds__(256) void cross_entropy_rows(LossArgs a)
     typedef float piece __attribute__((ext_vector_type(W)));
     constexpr int RPB = 256 / TPR;
     const int sub = threadIdx.x % TPR;
+    const float r = 1.0f / a.n;
     double sum = 0.0;
-    for (int row = blockIdx.x * RPB + threadIdx.x / TPR; row < a.rows; row += gridDim.x * RPB) {
+    piece xn[NV], tn[NV];  // the next row's
+    auto load = [&](int row) {
         const int64_t base = (int64_t)row * a.L;
-        piece x[NV], t[NV];
-        float m = -INFINITY;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int c = W * (TPR * j + sub);
-            if (c < a.L) {
-                x[j] = *(const piece *)(a.x + base + c);
-                t[j] = *(const piece *)(a.t + base + c);
+            if (row < a.rows && c < a.L) {
+                xn[j] = *(const piece *)(a.x + base + c);
+                tn[j] = *(const piece *)(a.t + base + c);
+            } else {
+                xn[j] = piece(-INFINITY);  // exp: 0
+                tn[j] = piece(0.0f);
             }
         }
+    };
+    const int stride = gridDim.x * RPB;
+    int row = blockIdx.x * RPB + threadIdx.x / TPR;
+    load(row);
+    for (; row < a.rows; row += stride) {
+        const int64_t base = (int64_t)row * a.L;
+        piece x[NV], t[NV], e[NV];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) x[j] = xn[j], t[j] = tn[j];
+        load(row + stride);
+        float m = -INFINITY;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            if (W * (TPR * j + sub) < a.L)
 #pragma unroll
-                for (int e = 0; e < W; ++e) m = fmaxf(m, x[j][e]);
+            for (int i = 0; i < W; ++i) m = fmaxf(m, x[j][i]);
         m = group_max<TPR>(m);
         float s = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            if (W * (TPR * j + sub) < a.L)
 #pragma unroll
-                for (int e = 0; e < W; ++e) {
-                    x[j][e] -= m;
-                    s += expf(x[j][e]);
-                }
-        const float logs = logf(group_sum<TPR>(s));
+            for (int i = 0; i < W; ++i) {
+                x[j][i] -= m;
+                e[j][i] = expf(x[j][i]);
+                s += W * (TPR * j + sub) < a.L ? e[j][i] : 0.0f;  // a row of -inf: NaN from its own elements only
+            }
+        s = group_sum<TPR>(s);
+        const float logs = logf(s), inv = 1.0f / s;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int c = W * (TPR * j + sub);
             if (c < a.L) {
                 piece p, g;
 #pragma unroll
-                for (int e = 0; e < W; ++e) {
+                for (int i = 0; i < W; ++i) {
                     float pe, ge;
-                    sum += (double)loss_element(x[j][e], logs, t[j][e], a.n, pe, ge);
-                    p[e] = pe, g[e] = ge;
+                    sum += (double)loss_element(x[j][i], logs, e[j][i], inv, t[j][i], a.n, r, pe, ge);
+                    p[i] = pe, g[i] = ge;
                 }
                 *(piece *)(a.probs + base + c) = p;
                 *(piece *)(a.grad + base + c) = g;
             }
         }
     }
-    store_partial(sum, a.partial);
+    store_sum(sum, a);
 }
 
 __global__ __launch_bounds__(256) void cross_entropy_long(LossArgs a)
 {
     __shared__ float red[4];
+    const float r = 1.0f / a.n;
     double sum = 0.0;
     for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
         const int64_t base = (int64_t)row * a.L;
@@ -295,15 +326,16 @@ __global__ __launch_bounds__(256) void cross_entropy_long(LossArgs a)
         for (int c = threadIdx.x; c < a.L; c += 256) m = fmaxf(m, x[c]);
         m = block_reduce<true>(m, red);
         for (int c = threadIdx.x; c < a.L; c += 256) s += expf(x[c] - m);
-        const float logs = logf(block_reduce<false>(s, red));
+        s = block_reduce<false>(s, red);
+        const float logs = logf(s), inv = 1.0f / s;
         for (int c = threadIdx.x; c < a.L; c += 256) {
             float p, g;
-            sum += (double)loss_element(x[c] - m, logs, t[c], a.n, p, g);
+            sum += (double)loss_element(x[c] - m, logs, expf(x[c] - m), inv, t[c], a.n, r, p, g);
             a.probs[base + c] = p;
             a.grad[base + c] = g;
         }
     }
-    store_partial(sum, a.partial);
+    store_sum(sum, a);
 }
 
 template <int TPR, int NV, int W>
@@ -359,7 +391,8 @@ extern "C" int cross_entropy_loss(const float *logits, const float *target, floa
     const int blocks = (int)std::min<int64_t>(((int64_t)rows + per_block - 1) / per_block, kLossBlocks);
     char *ws = (char *)scratch(kScratchSum, (size_t)blocks * sizeof(double) + 16);
     if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
-    const LossArgs a = {logits, target, probs, grad, (double *)ws, rows, L, n};
+    const HostSum result((uint64_t *)(ws + (size_t)blocks * sizeof(double)));
+    const LossArgs a = {logits, target, probs, grad, (double *)ws, result.out(), rows, L, n};
     if (L <= 16) launch_loss<16, 1, 1>(a, blocks);
     else if (L <= 32) launch_loss<32, 1, 1>(a, blocks);
     else if (by_block) hipLaunchKernelGGL(cross_entropy_long, dim3(blocks), dim3(256), 0, 0, a);
@@ -376,7 +409,5 @@ extern "C" int cross_entropy_loss(const float *logits, const float *target, floa
         else if (L <= 512) launch_loss<64, 8, 1>(a, blocks);
         else launch_loss<64, 16, 1>(a, blocks);
     }
-    if (!launch_ok("cross_entropy_loss")) return EMBER_ERR_DEVICE;
-    return sum_partials((double *)ws, blocks, (float *)(ws + (size_t)blocks * sizeof(double)), total,
-                        "cross_entropy_loss");
+    return launch_ok("cross_entropy_loss") ? result.read(total, "cross_entropy_loss") : EMBER_ERR_DEVICE;
 }
