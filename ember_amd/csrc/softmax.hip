@@ -255,8 +255,8 @@ __global__ __launch_bounds__(256) void cross_entropy_rows(LossArgs a)
     const float r = 1.0f / a.n;
     double sum = 0.0;
     piece xn[NV], tn[NV];  // the next row's
-    auto load = [&](int row) {
-        const int64_t base = (int64_t)row * a.L;
+    auto load = [&](int64_t row) {  // up to a stride past the last row, which may be 2^31 - 1
+        const int64_t base = row * a.L;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             const int c = W * (TPR * j + sub);
@@ -270,10 +270,10 @@ __global__ __launch_bounds__(256) void cross_entropy_rows(LossArgs a)
         }
     };
     const int stride = gridDim.x * RPB;
-    int row = blockIdx.x * RPB + threadIdx.x / TPR;
+    int64_t row = blockIdx.x * RPB + threadIdx.x / TPR;
     load(row);
     for (; row < a.rows; row += stride) {
-        const int64_t base = (int64_t)row * a.L;
+        const int64_t base = row * a.L;
         piece x[NV], t[NV], e[NV];
 #pragma unroll
         for (int j = 0; j < NV; ++j) x[j] = xn[j], t[j] = tn[j];
@@ -319,8 +319,8 @@ __global__ __launch_bounds__(256) void cross_entropy_long(LossArgs a)
     __shared__ float red[4];
     const float r = 1.0f / a.n;
     double sum = 0.0;
-    for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
-        const int64_t base = (int64_t)row * a.L;
+    for (int64_t row = blockIdx.x; row < a.rows; row += gridDim.x) {
+        const int64_t base = row * a.L;
         const float *x = a.x + base, *t = a.t + base;
         float m = -INFINITY, s = 0.0f;
         for (int c = threadIdx.x; c < a.L; c += 256) m = fmaxf(m, x[c]);

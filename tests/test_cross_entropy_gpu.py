@@ -98,3 +98,21 @@ def test_refuses_what_it_cannot_take():
         with pytest.raises(Exception):
             capi.check(L.cross_entropy_loss(None, None, None, None, rows, 4, 1.0, C.byref(total)), "cross_entropy_loss")
     assert L.cross_entropy_loss(None, None, None, None, 0, 4, 1.0, C.byref(total)) == 0
+
+
+def test_most_rows():
+    """2^31 - 1 rows of one class: the row indexes ahead of the last pass 2^31."""
+    rows, part = 2 ** 31 - 1, 1 << 20
+    L = capi.lib()
+    x, t, probs, grad = (DeviceArray((rows,)) for _ in range(4))
+    for a in (x, t, probs, grad):
+        L.hipMemset(C.c_void_p(a.ptr), 0, C.c_size_t(a.nbytes))
+    total = C.c_float(1)
+    capi.check(L.cross_entropy_loss(x.ptr, t.ptr, probs.ptr, grad.ptr, rows, 1, 2.0, C.byref(total)),
+               "cross_entropy_loss")
+    assert total.value == 0
+    for a, want in ((probs, 1), (grad, 0.5)):
+        for first in (0, rows // 2, rows - part):
+            got = np.empty(part, np.float32)
+            L.copy_from_device(got.ctypes.data, a.ptr + 4 * first, got.nbytes)
+            assert (got == want).all()
