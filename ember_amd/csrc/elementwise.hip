@@ -371,7 +371,7 @@ float sum(const float *a, int size)
     if (!ws) return 0.0f;
     double *partial = (double *)ws;
     uint64_t *res = (uint64_t *)(ws + (size_t)nblk * sizeof(double));
-    const ember::HostSum result(res);
+    const ember::HostSum result(res, false);
     hipLaunchKernelGGL(k_sum, dim3(nblk), dim3(kBlock), 0, 0, a, size, partial, result.out());
     if (!ember::launch_ok("sum")) return 0.0f;
     float host = 0.0f;
@@ -390,7 +390,7 @@ int mse_loss(const float *pred, const float *target, float *grad, int size, floa
     if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
     double *partial = (double *)ws;
     uint64_t *res = (uint64_t *)(ws + (size_t)nblk * sizeof(double));
-    const ember::HostSum result(res);
+    const ember::HostSum result(res, true);
     hipLaunchKernelGGL(k_mse, dim3(nblk), dim3(kBlock), 0, 0, pred, target, grad, scale, size, partial,
                        result.out());
     return ember::launch_ok("mse_loss") ? result.read(loss, "mse_loss") : EMBER_ERR_DEVICE;

@@ -3,9 +3,8 @@
 // memory, where the caller waits for it.  What this saves is latency: a kernel
 // of one workgroup, a device-to-host copy and the runtime's wait.  Measured, a
 // call that finds the device idle: sum of 1000 floats 20.5 -> 12.4 us, of 2^20
-// 20.7 -> 14.9, MSE over 2^20 18.3 -> 12.7.  (Waiting with
-// hipStreamSynchronize instead of polling: slower than the copy, the step of a
-// small classifier 107 against 87 us.)
+// 20.7 -> 14.9.  (Waiting with hipStreamSynchronize instead of polling is
+// slower than the copy: the step of a small classifier 107 against 87 us.)
 #pragma once
 
 #include "common.h"
@@ -73,10 +72,14 @@ __device__ __forceinline__ void finish_sum(double mine, double *partial, uint64_
 }  // namespace
 
 // Eight bytes of pinned host memory for a call's result, or, where there are
-// none, `res` in device memory.
+// none or the kernel also stores tensors, `res` in device memory.  The slot is
+// written while the kernel's other stores may still be in flight or in an L2,
+// and a caller may read its tensors on a stream of its own after the call:
+// such calls wait for the whole kernel with the copy (cross-entropy 8192 x 1000
+// 46 us; 37 without the wait, 58 polling and then hipStreamQuery until done).
 class HostSum {
 public:
-    explicit HostSum(uint64_t *res) : slot_(host_slot()), res_(res)
+    HostSum(uint64_t *res, bool stores_tensors) : slot_(stores_tensors ? nullptr : host_slot()), res_(res)
     {
         if (slot_) __atomic_store_n(slot_, 0, __ATOMIC_RELAXED);
     }

@@ -187,9 +187,8 @@ void launch_wave(const float *a, float *out, int rows, int L)
 // a workgroup each and three passes, of which the second and third hit the
 // caches.
 // Measured, value and gradient with the sum read back, composed and here: 8192
-// x 1000 179 and 37 us (the kernel 40 us without the next row's loads and with
-// a second expf and a division per element, 30 with them: 4.4 TB/s), 8192 x
-// 4096 688 and 137, 8192 x 1001 257 and 34, 64 x 10 60 and 14.
+// x 1000 179 and 46 us (the kernel 40 us without the next row's loads and with
+// a second expf and a division per element, 30 with them: 4.4 TB/s).
 constexpr int kLossBlocks = 1024;  // 4 workgroups of 4 waves per CU
 
 template <int TPR>
@@ -391,7 +390,7 @@ extern "C" int cross_entropy_loss(const float *logits, const float *target, floa
     const int blocks = (int)std::min<int64_t>(((int64_t)rows + per_block - 1) / per_block, kLossBlocks);
     char *ws = (char *)scratch(kScratchSum, (size_t)blocks * sizeof(double) + 16);
     if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
-    const HostSum result((uint64_t *)(ws + (size_t)blocks * sizeof(double)));
+    const HostSum result((uint64_t *)(ws + (size_t)blocks * sizeof(double)), true);
     const LossArgs a = {logits, target, probs, grad, (double *)ws, result.out(), rows, L, n};
     if (L <= 16) launch_loss<16, 1, 1>(a, blocks);
     else if (L <= 32) launch_loss<32, 1, 1>(a, blocks);
