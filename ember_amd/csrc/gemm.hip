@@ -12,12 +12,11 @@
 // Products run on the bf16 matrix cores at fp32 precision: every operand is
 // split exactly into three bf16 parts (split_bf16.h), and six of the nine
 // part products are accumulated in fp32.  One kernel covers every shape,
-// orientation and alignment; choose_shape picks its tile.
-#include <math.h>
-
+// orientation and alignment; choose_gemm (gemm_shape.h) picks its tile.
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_shape.h"
 #include "mfma.h"
 #include "split_bf16.h"
 
@@ -243,11 +242,11 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
     const int row0 = __builtin_amdgcn_readfirstlane((first + in_grp % rows_in_grp) * TM);
     const int col0 = __builtin_amdgcn_readfirstlane((in_grp / rows_in_grp) * TN);
 
-    int kbeg = 0, kend = g.k;
-    if (g.part) {
-        kbeg = blockIdx.z * g.kchunk;
-        kend = min(g.k, kbeg + g.kchunk);
-    }
+    // Slab 0 takes what k leaves over, the others are whole, so that the loop
+    // has no bounds on k and the short slab's guarded loads share the
+    // prologue's wait.
+    const KRange range = k_range(g.k, g.kchunk, blockIdx.z, BK);
+    const int kbeg = range.beg, kend = range.end, nslab = range.slabs, first_k = range.first;
     const float *A = g.a + (int64_t)blockIdx.y * g.sa;
     const float *B = g.b + (int64_t)blockIdx.y * g.sb;
 
@@ -264,11 +263,6 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
 
     OA oa;
     OB ob;
-    // Slab 0 takes what k leaves over, the others are whole, so that the loop
-    // has no bounds on k and the short slab's guarded loads share the
-    // prologue's wait.
-    const int nslab = (kend - kbeg + BK - 1) / BK;
-    const int first_k = kend - kbeg - (nslab - 1) * BK;
     const int arow = 32 * RB * wr + l32, bcol = 32 * CB * wc + l32;
     // Multiplies slab s (in as, bs) while slab s + 1 (in registers) is split
     // and stored to the other buffer and slab s + 2 is loaded.  Past the last
@@ -432,7 +426,7 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) acc[rb][cb] = zero16();
-            for (int k0 = kbeg; k0 < kend; k0 += 2) {
+            for (int64_t k0 = kbeg; k0 < kend; k0 += 2) {
                 const int64_t k = k0 + h32;
                 float av[RB], bv[CB];
 #pragma unroll
@@ -518,28 +512,11 @@ int num_cus()
 template <int TM, int TN, int WR, int WC, int BK, int PER_CU, bool TWO, bool TA, bool TB>
 void launch_tiles(GemmArgs &g, int batch, int ksplit)
 {
-    g.tiles_n = (g.n + TM - 1) / TM;
-    g.tiles_m = (g.m + TN - 1) / TN;
+    g.tiles_n = (int)ceil_div(g.n, TM);
+    g.tiles_m = (int)ceil_div(g.m, TN);
     hipLaunchKernelGGL((gemm_split_kernel<TM, TN, WR, WC, BK, PER_CU, TWO, TA, TB>),
                        dim3(g.tiles_n * g.tiles_m, batch, ksplit), dim3(64 * WR * WC), 0, 0, g);
 }
-
-// The three tiles, and what a launch with each costs: the 16-k steps of the
-// busiest CU, at the time one takes with the chip nearly empty (light_us: the
-// chain of waits of one tile) and full (full_us: throughput, and the clock
-// the power limit leaves), plus a launch's fixed cost.  Fitted to measured
-// times of 17 shapes with every tile and 1 to 8 splits (4096^3 down to
-// 17 x 33 x 5): the choice by this cost is the fastest of the measured ones
-// for 16 of them, 6 % off for one.  full_us as throughput: 256 x 256 tiles
-// 228 TFLOP/s at 4096^3 (128 x 128: 188), 128 x 128 181 TFLOP/s at
-// 8192 x 1024 x 1024 (64 x 64: 133, 256 x 256: 154); light_us: 12 products of
-// 197 x 333 x 250 11 us with 64 x 64, 17 with 128 x 128, 45 with 256 x 256.
-struct Shape {
-    int tm, tn, per_cu;
-    double full_us, light_us, fixed_us;
-};
-constexpr Shape kShapes[3] = {{256, 256, 1, 2.3, 1.75, 6.5}, {128, 128, 1, 0.73, 0.55, 4.5}, {64, 64, 3, 0.285, 0.36, 3.5}};
-constexpr int64_t kSplitBytes = int64_t(1) << 29;  // most scratch that splitting k may take
 
 template <bool TA, bool TB>
 void launch_shape(GemmArgs &g, int batch, int ksplit, int shape)
@@ -550,43 +527,6 @@ void launch_shape(GemmArgs &g, int batch, int ksplit, int shape)
         launch_tiles<128, 128, 4, 2, 32, 1, true, TA, TB>(g, batch, ksplit);
     else
         launch_tiles<64, 64, 2, 2, 32, 3, true, TA, TB>(g, batch, ksplit);
-}
-
-// k per split for `want` splits, a multiple of every tile's slab.
-int split_chunk(int k, int want)
-{
-    return ((k + want - 1) / want + 31) / 32 * 32;
-}
-
-// The cheapest tile and number of k splits.
-void choose_shape(const GemmArgs &g, int batch, int &shape, int &ksplit)
-{
-    const double cus = num_cus(), total = (double)batch * g.n * g.m;
-    double best = INFINITY;
-    for (int s = 0; s < 3; ++s) {
-        const Shape &p = kShapes[s];
-        const double tiles = (double)((g.n + p.tm - 1) / p.tm) * ((g.m + p.tn - 1) / p.tn) * batch;
-        for (int want : {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32, 48, 64}) {
-            if (want > 1 && (g.k / want < 64 || 4 * want * total > kSplitBytes)) break;
-            // The 256 x 256 tile sums all six part products together, the
-            // others keep the small ones apart and err a third as much: it
-            // splits k only as often as fills the chip, with short sums.
-            if (s == 0 && want > 1 && (want + 1) * tiles <= cus) continue;
-            const int chunk = want > 1 ? split_chunk(g.k, want) : g.k;
-            const int splits = want > 1 ? (g.k + chunk - 1) / chunk : 1;
-            const double work = tiles * splits, rounds = ceil(work / cus), steps = (chunk + 15) / 16;
-            const double step_us = p.per_cu > 1
-                                       ? fmax(p.light_us, p.full_us * rounds)
-                                       : rounds * (p.light_us + (p.full_us - p.light_us) * fmin(1.0, work / cus));
-            double us = p.fixed_us + steps * step_us;
-            if (splits > 1) us += 3.0 + (2 * splits + 1) * 4 * total / 5e6;  // the reduction's launch and bytes
-            if (us < best) {
-                best = us;
-                shape = s;
-                ksplit = splits;
-            }
-        }
-    }
 }
 
 int gemm_launch(const float *a, const float *b, float *out, int batch, int n, int m, int k,
@@ -621,13 +561,14 @@ int gemm_launch(const float *a, const float *b, float *out, int batch, int n, in
     g.pre = pre;
     g.act = act;
 
-    int shape = 2, ksplit = 1;
-    choose_shape(g, batch, shape, ksplit);
+    const GemmChoice choice = choose_gemm(n, m, k, batch, num_cus());
+    const int shape = choice.shape;
+    int ksplit = choice.ksplit;
     const int64_t total = (int64_t)batch * n * m;
     if (ksplit > 1) {
         g.part = (float *)scratch(kScratchGemmSplit, (size_t)ksplit * total * sizeof(float), true);
         if (g.part)
-            g.kchunk = split_chunk(k, ksplit);
+            g.kchunk = (int)choice.kchunk;
         else
             ksplit = 1;  // no memory for the parts: one sum per element
     }

@@ -4,6 +4,8 @@ values the split cannot carry (infinities, NaN, magnitudes next to the largest
 float, rows below 2^-100), and its error against float64 next to the fp32
 chain's."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -127,3 +129,20 @@ def test_sums_over_rows_and_columns_are_unbiased(n, k, m, fp32_chain):
 def test_zero_products_give_positive_zero():
     a, b = _u((70, 40), 13), np.zeros((40, 90), np.float32)
     assert not np.signbit(G.gemm_ex(a, b)).any()
+
+
+@pytest.mark.parametrize("k", [1431655765, 1500000001, 2 ** 31 - 1])
+def test_longest_sums(k):
+    """A dot product whose k, in chunks and slabs, passes 2^31: zeros but for
+    whole numbers at the ends, about every split's likely ends and 2^30."""
+    at = np.unique(np.clip(np.r_[0:40, k - 40:k, 2 ** 30 - 20:2 ** 30 + 20,
+                                 np.concatenate([np.arange(-2, 34) + k * z // 64 for z in range(64)])], 0, k - 1))
+    a = capi.DeviceArray((k,))
+    one, out = np.ones(1, np.float32), capi.DeviceArray((1,))
+    L = capi.lib()
+    assert L.hipMemset(C.c_void_p(a.ptr), 0, C.c_size_t(a.nbytes)) == 0
+    for i in at:
+        L.copy_to_device(a.ptr + 4 * int(i), one.ctypes.data, 4)
+    for ta, tb in ((0, 0), (1, 1)):
+        capi.check(L.gemm_ex(a.ptr, a.ptr, out.ptr, 1, 1, 1, k, ta, tb, None, None, None, 0), "gemm_ex")
+        assert out.numpy()[0] == len(at)
