@@ -13,6 +13,7 @@
 // split exactly into three bf16 parts (split_bf16.h), and six of the nine
 // part products are accumulated in fp32.  One kernel covers every shape,
 // orientation and alignment; choose_gemm (gemm_shape.h) picks its tile.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -31,6 +32,7 @@ struct GemmArgs {
     int ta, tb;          // a stored k x n / b stored m x k
     int64_t sa, sb, sc;  // batch strides (elements)
     int tiles_n, tiles_m;
+    int tile0;           // first tile of this launch
     int kchunk;          // split-K: k range of one blockIdx.z (multiple of 32)
     float *part;         // split-K partial sums [ksplit][batch][n][m]
     // Epilogue (all optional): out = act(acc + bias[col]) + residual, with
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
     const int wr = w / WC, wc = w % WC;
 
     const int ntiles = g.tiles_n * g.tiles_m;
-    int tile = blockIdx.x;
+    int tile = g.tile0 + blockIdx.x;
     if (ntiles % 8 == 0) tile = (tile % 8) * (ntiles / 8) + tile / 8;
     constexpr int GROUP = 8;
     const int per_group = GROUP * g.tiles_m;
@@ -514,8 +516,13 @@ void launch_tiles(GemmArgs &g, int batch, int ksplit)
 {
     g.tiles_n = (int)ceil_div(g.n, TM);
     g.tiles_m = (int)ceil_div(g.m, TN);
-    hipLaunchKernelGGL((gemm_split_kernel<TM, TN, WR, WC, BK, PER_CU, TWO, TA, TB>),
-                       dim3(g.tiles_n * g.tiles_m, batch, ksplit), dim3(64 * WR * WC), 0, 0, g);
+    static_assert(kTilesPerLaunch % 8 == 0 && kTilesPerLaunch * 64 * WR * WC < int64_t(1) << 32, "threads of a grid in x");
+    const int64_t tiles = (int64_t)g.tiles_n * g.tiles_m;
+    for (int64_t t0 = 0; t0 < tiles; t0 += kTilesPerLaunch) {
+        g.tile0 = (int)t0;
+        hipLaunchKernelGGL((gemm_split_kernel<TM, TN, WR, WC, BK, PER_CU, TWO, TA, TB>),
+                           dim3((unsigned)std::min(tiles - t0, kTilesPerLaunch), batch, ksplit), dim3(64 * WR * WC), 0, 0, g);
+    }
 }
 
 template <bool TA, bool TB>

@@ -29,6 +29,10 @@ constexpr GemmShape kGemmShapes[3] = {
     {256, 256, 1, 2.3, 1.75, 6.5}, {128, 128, 1, 0.73, 0.55, 4.5}, {64, 64, 3, 0.285, 0.36, 3.5}};
 constexpr int64_t kSplitBytes = int64_t(1) << 29;  // most scratch that splitting k may take
 
+// A grid holds fewer than 2^32 threads in x, which thin outputs of more than
+// 2^30 rows or columns pass: the rest goes in further launches.
+constexpr int64_t kTilesPerLaunch = int64_t(1) << 22;
+
 // k per split for `want` splits, a multiple of every tile's slab.
 inline int64_t split_chunk(int64_t k, int want) { return ceil_div(ceil_div(k, want), 32) * 32; }
 

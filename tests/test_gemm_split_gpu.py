@@ -146,3 +146,21 @@ def test_longest_sums(k):
     for ta, tb in ((0, 0), (1, 1)):
         capi.check(L.gemm_ex(a.ptr, a.ptr, out.ptr, 1, 1, 1, k, ta, tb, None, None, None, 0), "gemm_ex")
         assert out.numpy()[0] == len(at)
+
+
+@pytest.mark.parametrize("size", [2 ** 30 + 1, 1100000000, 2 ** 31 - 200, 2 ** 31 - 1])
+@pytest.mark.parametrize("rows", [True, False])
+def test_longest_outputs(size, rows):
+    """One column or row of more tiles than one grid holds threads for."""
+    L = capi.lib()
+    a, b, out = capi.DeviceArray((size,)), capi.DeviceArray((1,), np.full(1, 3, np.float32)), capi.DeviceArray((size,))
+    n, m = (size, 1) if rows else (1, size)
+    assert L.hipMemset(C.c_void_p(a.ptr), 0x40, C.c_size_t(a.nbytes)) == 0
+    assert L.hipMemset(C.c_void_p(out.ptr), 0, C.c_size_t(out.nbytes)) == 0
+    x, y = (a, b) if rows else (b, a)
+    for k, want in ((1, 3 * np.full(1, 0x40404040, np.uint32).view(np.float32)[0]), (0, 0)):
+        capi.check(L.gemm_ex(x.ptr, y.ptr, out.ptr, 1, n, m, k, 0, 0, None, None, None, 0), "gemm_ex")
+        part = np.empty(min(size, 1 << 22), np.float32)
+        for first in (0, size // 2, 2 ** 30 - len(part), size - len(part)):
+            L.copy_from_device(part.ctypes.data, out.ptr + 4 * first, part.nbytes)
+            assert (part == want).all()
