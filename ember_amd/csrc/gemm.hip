@@ -85,8 +85,7 @@ struct Operand {
     unsigned voff;      // !KC: this lane's byte offset from there
     int kq[G];          // the group's k offset within the slab
     float v[G][8];
-    unsigned bits[G];   // OR of the group's elements so far (split_tiny)
-    unsigned neg[G];    // sign_of the group's row
+    float f[G];         // kSplitScale with sign_of the group's row
     unsigned s[G][3][2];  // two split pairs: hi, mid, lo
 
     static __device__ __forceinline__ int unit(int r, int q)
@@ -114,10 +113,9 @@ struct Operand {
             int q = unit_of(tid, g);
             if (!KC) q = __builtin_amdgcn_readfirstlane(q);  // one k row per wave: scalar addresses
             kq[g] = 8 * q;
-            neg[g] = sign_of(row0 + row_of(tid, g));
+            f[g] = flip(kSplitScale, sign_of(row0 + row_of(tid, g)));
             p[g] = KC ? base + (int64_t)(row0 + r) * ld + kbeg + 8 * q : base + (int64_t)(kbeg + 8 * q) * ld + row0;
             if (!KC) voff = 4u * (unsigned)r;
-            bits[g] = 0;
         }
     }
     __device__ __forceinline__ float at(int g, int j, int64_t ld) const
@@ -161,9 +159,7 @@ struct Operand {
     // each plane is stored.
     __device__ __forceinline__ void split_store(int g, int i, u32x4 *__restrict__ lds, int tid)
     {
-        const float x = flip(v[g][2 * i], neg[g]), y = flip(v[g][2 * i + 1], neg[g]);
-        bits[g] |= float_bits(v[g][2 * i]) | float_bits(v[g][2 * i + 1]);
-        split_pair(x, y, s[g][0][i & 1], s[g][1][i & 1], s[g][2][i & 1]);
+        split_pair(v[g][2 * i] * f[g], v[g][2 * i + 1] * f[g], s[g][0][i & 1], s[g][1][i & 1], s[g][2][i & 1]);
         if (i & 1) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
             u32x2 *const to = (u32x2 *)lds + 2 * unit(row_of(tid, g), unit_of(tid, g)) + i / 2;
@@ -178,26 +174,14 @@ struct Operand {
 #pragma unroll
             for (int i = 0; i < 4; ++i) split_store(g, i, lds, tid);
     }
-    __device__ __forceinline__ bool tiny() const
-    {
-        bool t = false;
-#pragma unroll
-        for (int g = 0; g < G; ++g) t |= split_tiny(bits[g]);
-        return t;
-    }
-    __device__ __forceinline__ void row_bits(unsigned *m, int tid) const
-    {
-#pragma unroll
-        for (int g = 0; g < G; ++g) atomicOr(&m[row_of(tid, g)], bits[g]);
-    }
 };
 
 // A TM x TN block of out per workgroup of WR x WC waves, each 32*RB x 32*CB.
 // What bounds it: the matrix cores, and at 4096^3 the power limit with them
 // (72 % of cycles busy, at 1.70 GHz; the same launch on constant operands
 // holds 2.28 GHz): 933 -> 601 us, 147 -> 228 TFLOP/s against the fp32
-// instruction's kernel this replaced.  Splitting costs 5.5 vector operations
-// per element staged (2.2 per matrix instruction in the 256 x 256 tile, 4 are
+// instruction's kernel this replaced.  Splitting costs 6.5 vector operations
+// per element staged (2.6 per matrix instruction in the 256 x 256 tile, 4 are
 // free beside one), so operands are split once, when they enter LDS, and not
 // by each wave that reads them.
 //   * k is walked in slabs of BK through two LDS buffers, one barrier per
@@ -209,9 +193,8 @@ struct Operand {
 //   * split-K (g.part): blockIdx.z walks k in [z*kchunk, (z+1)*kchunk) and
 //     stores its raw sums to part; gemm_splitk_reduce adds the splits in
 //     order and applies the epilogue, so results do not depend on timing.
-//   * a wave whose sums are not finite, or whose workgroup met a row too
-//     small to split (split_bf16.h), computes its block again from global
-//     memory with the fp32 instruction.
+//   * a wave whose sums are not finite (split_bf16.h) computes its block
+//     again from global memory with the fp32 instruction.
 template <int TM, int TN, int WR, int WC, int BK, int PER_CU, bool TWO, bool TA, bool TB>
 __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmArgs g)
 {
@@ -222,7 +205,6 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
     
     __shared__ u32x4 As0[3 * OA::kPlane], As1[3 * OA::kPlane];
     __shared__ u32x4 Bs0[3 * OB::kPlane], Bs1[3 * OB::kPlane];
-    __shared__ int tiny_row;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -335,7 +317,6 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
         ob.advance(g.ldb, k);
     };
 
-    if (tid == 0) tiny_row = 0;
     if (nslab > 0) {
         oa.init(A, g.lda, row0, g.n, kbeg, tid);
         ob.init(B, g.ldb, col0, g.m, kbeg, tid);
@@ -383,25 +364,8 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
 
     // Anything the split cannot carry (see split_bf16.h): do this wave's
     // block again with the fp32 instruction.
+    float unscale = 1.0f / (kSplitScale * kSplitScale);
     if (nslab > 0) {
-        if (oa.tiny() || ob.tiny()) tiny_row = 1;
-        __syncthreads();
-        if (tiny_row) {
-            // A thread saw only its share of a row's k: take the row's whole.
-            unsigned *const ma = (unsigned *)As0, *const mb = (unsigned *)Bs0;
-            for (int i = tid; i < TM; i += NT) ma[i] = 0;
-            for (int i = tid; i < TN; i += NT) mb[i] = 0;
-            __syncthreads();
-            oa.row_bits(ma, tid);
-            ob.row_bits(mb, tid);
-            if (tid == 0) tiny_row = 0;
-            __syncthreads();
-            bool tiny = false;
-            for (int i = tid; i < TM; i += NT) tiny |= split_tiny(ma[i]);
-            for (int i = tid; i < TN; i += NT) tiny |= split_tiny(mb[i]);
-            if (tiny) tiny_row = 1;
-            __syncthreads();
-        }
         float probe = 0.0f;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -409,7 +373,8 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
             for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) probe = fmaf(acc[rb][cb][i], 0.0f, probe);
-        if (__ballot(probe != 0.0f) != 0 || tiny_row) {
+        if (__ballot(probe != 0.0f) != 0) {
+            unscale = 1.0f;
             const float *ap[RB], *bp[CB];
             unsigned aneg[RB], bneg[CB];
 #pragma unroll
@@ -466,10 +431,9 @@ __global__ __launch_bounds__(64 * WR * WC, PER_CU) void gemm_split_kernel(GemmAr
                 const int row = row0 + 32 * (RB * wr + rb) + acc_row(i, el >> 5);
                 if (row >= g.n) continue;
                 const int64_t off = (int64_t)row * g.m + col;
-                // The sign comes off by a multiplication (bits of an
-                // accumulator flipped as an integer make the compiler spill),
-                // and a zero sum stays +0.
-                float v = fmaf(acc[rb][cb][i], flip(1.0f, sign_of(row) ^ sign_of(col)), 0.0f);
+                // Scale and sign come off by a multiplication, and a zero
+                // sum stays +0.
+                float v = fmaf(acc[rb][cb][i], flip(unscale, sign_of(row) ^ sign_of(col)), 0.0f);
                 if (epi) {
                     // out = act(acc + bias) + residual, pre = acc + bias.
 #pragma clang fp contract(off)

@@ -3,18 +3,21 @@
 //
 // x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi -
 // mid), each rounded to nearest: 3 x 8 bits hold the 24 bits of an fp32
-// significand, so the sum is x itself (for |x| >= 2^-109, where lo is still
-// a bf16 number, and below bf16's largest value).  A product a*b is then
+// significand, so the sum is x itself, down to bf16's smallest number, 2^-133.
+// fp32's is 2^-149: operands are multiplied by 2^16 (kSplitScale) as they are
+// split, so that every fp32 number below 2^111 is split exactly, denormal ones
+// too (the matrix core keeps denormal operands and sums, measured), and the
+// results carry 2^32.  A product a*b is then
 //   lo*hi' + hi*lo' + mid*mid' + mid*hi' + hi*mid' + hi*hi'
-// with each part product exact in the matrix core; the three left out are
-// below 2^-26 |a b|, less than the 2^-24 that one fp32 rounding costs.  The
-// small terms are added first.  v_mfma_f32_32x32x16_bf16 does 32 times the
-// work of v_mfma_f32_32x32x2f32 per instruction in half its time (8 against
-// 16 passes), so six of them are 2.67 times as fast, and they round the
-// accumulator 6 times per 16 products where the fp32 instruction does it 8
-// times.  Measured against float64 (relative 2-norm error, N(0,1) operands):
-// K = 64 1.1e-7 (fp32 instruction 1.4e-7), K = 4096 1.0e-6 (1.2e-6); U(0,1):
-// K = 4096 5.3e-7 (8.6e-7).
+// with each part product exact in the matrix core; the three left out are at
+// most 2^-24 |a b| together, one fp32 rounding (mid up to 2^-8 of x, lo up to
+// 2^-17), and mostly far below it.  The small terms are added first.
+// v_mfma_f32_32x32x16_bf16 does 8 times the work of v_mfma_f32_32x32x2f32 per
+// instruction in half its time (8 against 16 passes), so six of them are 2.67
+// times as fast, and they round the accumulator 6 times per 16 products where
+// the fp32 instruction does it 8 times.  Measured against float64 (relative
+// 2-norm error, N(0,1) operands): K = 64 1.1e-7 (fp32 instruction 1.4e-7),
+// K = 4096 1.0e-6 (1.2e-6); U(0,1): K = 4096 5.3e-7 (8.6e-7).
 //
 // The matrix core rounds down, not to nearest, what it shifts out when it
 // lines a sum's terms up: -0.004 ulp of the sum per instruction, and up to a
@@ -28,9 +31,9 @@
 // instruction 1.1e-6, split 1.3e-5, split with signs 9.5e-7.
 //
 // What the split cannot carry is caught by the kernels that use it and
-// computed again with the fp32 instruction: infinities and values that round
-// up to one (their remainder is NaN, so an accumulator that holds them is not
-// finite), and rows so small that bf16 has no bits left for lo.
+// computed again with the fp32 instruction: infinities, values from 2^111 on
+// and sums from 2^96 on (a part or its remainder is infinite or NaN, so an
+// accumulator that holds it is not finite).
 //
 // Operands of v_mfma_f32_32x32x16_bf16: lane l holds row (or column) l % 32
 // and the 8 contraction elements of its half l / 32, as four packed pairs.
@@ -46,6 +49,8 @@ namespace ember {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr float kSplitScale = 0x1p16f;
 
 // A row whose largest magnitude is below 2^-95 (and not 0) is left to the
 // fp32 instruction, so that a row that stays keeps lo down to 2^-39 of its

@@ -1,7 +1,7 @@
 """The split-bf16 GEMM where it can go wrong: tile edges and short last k-slabs
 of each tile shape and orientation, operands that do not start on 16 bytes,
 values the split cannot carry (infinities, NaN, magnitudes next to the largest
-float, rows below 2^-100), and its error against float64 next to the fp32
+float), elements of every magnitude beside larger ones, and its error against float64 next to the fp32
 chain's."""
 
 import ctypes as C
@@ -25,10 +25,11 @@ def _stored(x, trans):
 
 def _bound(a, b):
     """6 roundings per 16 products of partial sums of at most |a||b|, and the
-    part products left out (2^-25 of |a||b|)."""
+    part products left out: mid up to 2^-8 and lo up to 2^-17 of an element,
+    so 2 * 2^-25 + 2^-34 of |a||b|, rounded up."""
     k = a.shape[1]
     mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
-    return (0.375 * k + 8) * 2.0 ** -24 * mag + 2.0 ** -25 * mag
+    return (0.375 * k + 8) * 2.0 ** -24 * mag + 2.0 ** -23 * mag
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
@@ -164,3 +165,33 @@ def test_longest_outputs(size, rows):
         for first in (0, size // 2, 2 ** 30 - len(part), size - len(part)):
             L.copy_from_device(part.ctypes.data, out.ptr + 4 * first, part.nbytes)
             assert (part == want).all()
+
+
+@pytest.mark.parametrize("small,large", [(-95, 60), (-112, 90), (-120, 100), (-126, 100), (-135, 110), (-145, 100)])
+@pytest.mark.parametrize("n,k,m", [(90, 200, 75), (700, 96, 600), (4096, 40, 4096)])
+@pytest.mark.parametrize("swap", [False, True])
+def test_small_elements_beside_large_ones(n, k, m, small, large, swap):
+    """Elements that bf16 alone has few bits for, in rows whose other elements
+    are ordinary and meet zeros: each output keeps fp32's precision.  (In fp32
+    the small ones are denormal from 2^-127 on: exact inputs, fewer bits.)"""
+    a, b = _u((n, k), 14), _u((k, m), 15)
+    a[:, ::2] *= np.float32(2.0 ** small)
+    b[::2] = np.ldexp(b[::2], large)
+    b[1::2, : m // 2] = 0
+    b[1::2, m // 2:] *= np.float32(2.0 ** -40)
+    if swap:
+        a, b = np.ascontiguousarray(b.T), np.ascontiguousarray(a.T)
+    rows = np.arange(0, a.shape[0], max(1, a.shape[0] // 64))
+    ref = a[rows].astype(np.float64) @ b.astype(np.float64)
+    assert (np.abs(G.gemm_ex(a, b)[rows] - ref) <= _bound(a[rows], b) + 2.0 ** -149 * k).all()
+
+
+@pytest.mark.parametrize("ea,eb", [(-60, -60), (-70, -64), (-100, -40), (100, -100), (115, -120), (-130, 115), (60, 50)])
+def test_magnitudes_of_operands(ea, eb):
+    """Products that are small themselves, and operands of 2^111 and sums of
+    2^96 and more, which the scaled split leaves to the fp32 instruction."""
+    n, k, m = 130, 100, 90
+    a, b = np.ldexp(_u((n, k), 16), ea), np.ldexp(_u((k, m), 17), eb)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    # Denormal results round at 2^-149, once per sum or part of it.
+    assert (np.abs(G.gemm_ex(a, b) - ref) <= _bound(a, b) + 2.0 ** -149 * k).all()
