@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
     constexpr int DB = D / 32, KS = D / 16, KB = T::KB, NT = T::NT, G = T::G;
     constexpr int PF = D == 128 && NW == 8 ? 1 : 2;  // K operand register sets
     __shared__ u32x4 Ks[2 * T::BUF], Vs[2 * T::BUF];
-    __shared__ int tiny_v;
+    __shared__ int big;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -154,6 +154,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
     const int b = bh / a.H;
     const int hh = bh - b * a.H;
     const int S = a.S;
+    constexpr float kBig = 0x1p44f * kSplitScale;
+    const float c = a.c / (kSplitScale * kSplitScale);
     const int64_t in_base = (int64_t)b * a.in_sb + (int64_t)hh * a.in_sh;
     const float *__restrict__ kbase = a.k + in_base;
     const float *__restrict__ vbase = a.v + in_base;
@@ -167,7 +169,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
         const int m0 = second ? BQ * (a.nqb - 1 - qb) + 32 * (w - NW / 2) : q0 + 32 * (w >= 4 ? 11 - w : w);
         const bool idle = second && qb == a.nqb - 1 - qb;  // an odd nqb's middle block is alone
         const int mq = m0 + l32;
-        const unsigned sgn = sign_of(mq);
+        // O^T's columns carry 2^32 and the query's sign (split_bf16.h).
+        const float pscale = flip(kSplitScale, sign_of(mq));
         const int kend = CAUSAL ? min(S, q0 + BQ) : S;
         const int ntiles = (kend + T::KEYS - 1) / T::KEYS;
 
@@ -178,9 +181,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
 
         // ---- staging ----
         float kreg[G][8], vreg[G][8];
-        unsigned vbits[G];  // OR of the V elements staged (split_tiny)
-#pragma unroll
-        for (int g = 0; g < G; ++g) vbits[g] = 0;
+        float top = 0.0f;  // largest magnitude of the Q and K elements split, scaled
         auto load_k = [&](int n0, int g) {
             const int i = ti + NT * g, r = i / T::UK, u = i % T::UK;
             const float *src = kbase + (int64_t)min(n0 + r, S - 1) * a.in_ss + 8 * u;
@@ -203,10 +204,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
         // Pair i (of 4) of group g of K (v = false) or V; every second one
         // stores half a unit of each plane.
         auto split_store = [&](bool v, int g, int i, u32x4 *kn, u32x4 *vn) {
-            const float x = v ? vreg[g][2 * i] : kreg[g][2 * i], y = v ? vreg[g][2 * i + 1] : kreg[g][2 * i + 1];
-            if (v) {
-                vbits[g] |= float_bits(x) | float_bits(y);
-                asm volatile("" : "+v"(vbits[g]));  // here, so that x and y die here
+            const float x = (v ? vreg[g][2 * i] : kreg[g][2 * i]) * kSplitScale;
+            const float y = (v ? vreg[g][2 * i + 1] : kreg[g][2 * i + 1]) * kSplitScale;
+            if (!v) {
+                top = fmaxf(top, fmaxf(fabsf(x), fabsf(y)));
+                asm volatile("" : "+v"(top));  // here, so that x and y die here
             }
             split_pair(x, y, part[0][i & 1], part[1][i & 1], part[2][i & 1]);
             if (i & 1) {
@@ -244,11 +246,14 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
                 float x[8];
                 const f32x4 t0 = *(const f32x4 *)(src + 16 * ks), t1 = *(const f32x4 *)(src + 16 * ks + 4);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = t0[j], x[4 + j] = t1[j];
+                for (int j = 0; j < 4; ++j) x[j] = t0[j] * kSplitScale, x[4 + j] = t1[j] * kSplitScale;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) top = fmaxf(top, fabsf(x[j]));
                 qf[ks] = split8(x);
             }
         }
-        if (tid == 0) tiny_v = 0;
+        asm volatile("" : "+v"(top));
+        if (tid == 0) big = a.c > 0.0f && a.c < 0x1p-94f;  // c below would be denormal
         stage_all(Ks, Vs, tile_n0(1));
         __syncthreads();
 
@@ -314,7 +319,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
             // otherwise exceed it by more than 2^8: the result is the same
             // softmax, and most tiles skip the rescale of O.  Tile 0 holds
             // key 0, visible to every query, so it sets a finite mrun.
-            const float tm2 = tmax * a.c;
+            const float tm2 = tmax * c;
             if (__ballot(tm2 > mrun + 8.0f) != 0) {
                 const float mnew = fmaxf(mrun, tm2);
                 const float alpha = __builtin_amdgcn_exp2f(mrun - mnew);
@@ -332,7 +337,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const float sv = sacc[blk][i];
-                        sacc[blk][i] = sv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(sv, a.c, -mrun));
+                        sacc[blk][i] = sv == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(sv, c, -mrun));
                         tsum += sacc[blk][i];
                     }
             } else {
@@ -340,18 +345,18 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
                 for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
-                        sacc[blk][i] = __builtin_amdgcn_exp2f(fmaf(sacc[blk][i], a.c, -mrun));
+                        sacc[blk][i] = __builtin_amdgcn_exp2f(fmaf(sacc[blk][i], c, -mrun));
                         tsum += sacc[blk][i];
                     }
             }
-            // P^T's parts, with the query's sign (split_bf16.h).
+            // P^T's parts, with the query's sign.
 #pragma unroll
             for (int blk = 0; blk < KB; ++blk)
 #pragma unroll
                 for (int i = 0; i < 16; i += 2) {
                     Split8 &f = pf[2 * blk + i / 8];
                     unsigned h, m, l;
-                    split_pair(flip(sacc[blk][i], sgn), flip(sacc[blk][i + 1], sgn), h, m, l);
+                    split_pair(sacc[blk][i] * pscale, sacc[blk][i + 1] * pscale, h, m, l);
                     f.part[0][i / 2 % 4] = h;
                     f.part[1][i / 2 % 4] = m;
                     f.part[2][i / 2 % 4] = l;
@@ -394,10 +399,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
             __syncthreads();
         }
 
-        bool tiny = false;
-#pragma unroll
-        for (int g = 0; g < G; ++g) tiny |= split_tiny(vbits[g]);
-        if (tiny) tiny_v = 1;
+        // Q and K below 2^44: no score passes 2^95, with its scale fp32's
+        // largest number.  (V and the weights show in O.)
+        if (top >= kBig) big = 1;
         __syncthreads();
         const float ltot = lrun + __shfl_xor(lrun, 32);
         float probe = ltot * 0.0f;
@@ -406,10 +410,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
 #pragma unroll
             for (int i = 0; i < 16; ++i) probe = fmaf(oacc[db][i], 0.0f, probe);
         if (idle) {
-        } else if (__ballot(probe != 0.0f) != 0 || tiny_v) {
+        } else if (__ballot(probe != 0.0f) != 0 || big) {
             rows_f32<D, CAUSAL>(a, b, hh, bh, m0);
         } else if (mq < S) {
-            const float inv = flip(1.0f / ltot, sgn);
+            const float inv = 1.0f / (kSplitScale * kSplitScale) / (ltot * pscale) * kSplitScale;
             float *orow = a.o + (int64_t)b * a.out_sb + (int64_t)hh * a.out_sh + (int64_t)mq * a.out_ss;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
@@ -422,7 +426,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 && D < 128 ? 3 : 1) void attn_fwd_
                 }
             if (h32 == 0) a.lse[(int64_t)bh * S + mq] = (mrun + log2f(ltot)) * kLn2;
         }
-        if (BLOCKS == kTurn) __syncthreads();  // tiny_v and the buffers, before the next block
+        if (BLOCKS == kTurn) __syncthreads();  // big and the buffers, before the next block
     };
 
     if constexpr (BLOCKS == kTurn) {

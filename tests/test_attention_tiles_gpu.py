@@ -1,7 +1,8 @@
 """The split-bf16 forward (attn_fwd_kernel) where it can go wrong: lengths
 around its key tiles and query blocks in each launch form (4 or 8 waves, one
-block, two at once, two in turn), values that the split cannot carry, and its
-error against float64 next to the fp32 instruction's."""
+block, two at once, two in turn), values that the split cannot carry, operands
+of every magnitude, and its error against float64 next to the fp32
+instruction's."""
 
 import numpy as np
 import pytest
@@ -11,12 +12,12 @@ import gpu_helpers as G
 pytestmark = pytest.mark.gpu
 
 
-def _ref(q, k, v, causal):
+def _ref(q, k, v, causal, scale=None):
     """float64 O and LSE of (S, D) operands; a score of -inf is a weight of 0."""
     q, k, v = (x.astype(np.float64) for x in (q, k, v))
     S, D = q.shape
     with np.errstate(invalid="ignore", over="ignore"):
-        s = q @ k.T * np.float64(np.float32(1 / np.sqrt(D)))
+        s = q @ k.T * np.float64(np.float32(1 / np.sqrt(D) if scale is None else scale))
     if causal:
         s[np.triu(np.ones((S, S), bool), 1)] = -np.inf
     m = s.max(-1, keepdims=True)
@@ -99,6 +100,56 @@ def test_tiny_values_keep_their_precision(H, S, D, causal, exponent):
     for h in (0, H - 1):
         ro, _ = _ref(q[0, h], k[0, h], v[0, h], causal)
         np.testing.assert_allclose(o[0, h] * 2.0 ** -exponent, ro * 2.0 ** -exponent, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("eq,ek,es", [(-122, 122, 0), (122, -122, 0), (-120, 40, 80), (40, -130, 90), (-60, -60, 120),
+                                      (100, -140, 40), (60, 40, -100), (20, 20, -40)])
+def test_scores_of_small_and_large_operands(H, S, D, causal, eq, ek, es):
+    """Q and K of 2^eq and 2^ek, denormal ones too, which the scale 2^es
+    brings back to ordinary scores: O and LSE to fp32 precision."""
+    q, k, v = _qkv(H, S, D, 5)
+    q, k, scale = np.ldexp(q, eq), np.ldexp(k, ek), np.ldexp(1 / np.sqrt(D), es)
+    o, lse = G.attention_fwd(q, k, v, causal, scale)
+    for h in (0, H - 1):
+        ro, rl = _ref(q[0, h], k[0, h], v[0, h], causal, scale)
+        # A score is the sum of D products of a few units: 2^-24 of some D.
+        np.testing.assert_allclose(o[0, h], ro, rtol=0, atol=2.0 ** -22 * np.sqrt(D))
+        np.testing.assert_allclose(lse[0, h], rl, rtol=0, atol=2.0 ** -22 * np.sqrt(D))
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("exponent", [-112, -120, -125])
+def test_tiny_values_beside_large_ones_of_no_weight(H, S, D, causal, exponent):
+    """Small V rows keep their precision next to large ones that a query gives
+    no weight, or (causal) does not see."""
+    q, k, v = _qkv(H, S, D, 6)
+    v *= np.float32(2.0 ** exponent)
+    q[..., 0], k[..., 0] = 8, 0
+    k[:, :, 20:S:7, 0] = -2000                         # weight exp(-1400) at most: 0
+    v[:, :, 20:S:7] = 1e6
+    o, _ = G.attention_fwd(q, k, v, causal)
+    for h in (0, H - 1):
+        ro, _ = _ref(q[0, h], k[0, h], v[0, h], causal)
+        size, _ = _ref(q[0, h], k[0, h], np.abs(v[0, h]), causal)
+        assert (np.abs(o[0, h] - ro) <= 1e-5 * size + 2.0 ** -148).all()
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+def test_tiny_weights_of_large_values(H, S, D, causal):
+    """Weights of exp(-86), 2^-124, beside one of 1 whose V is 0."""
+    q, k, v = (np.zeros((1, H, S, D), np.float32) for _ in range(3))
+    rng = np.random.default_rng(7)
+    q[..., 0] = np.sqrt(D)
+    k[:, :, 1:, 0] = rng.uniform(-86.4, -85, (1, H, S - 1)).astype(np.float32)
+    v[:, :, 1:] = np.ldexp(rng.uniform(-1, 1, (1, H, S - 1, D)).astype(np.float32), 60)
+    o, _ = G.attention_fwd(q, k, v, causal)
+    for h in (0, H - 1):
+        ro, _ = _ref(q[0, h], k[0, h], v[0, h], causal)
+        size, _ = _ref(q[0, h], k[0, h], np.abs(v[0, h]), causal)
+        # The exponent, about 124 in base 2, has an ulp of 2^-17: 2^-18 ln 2
+        # each in the product with the scale and in the sum with the maximum.
+        assert (np.abs(o[0, h] - ro) <= 2.0 ** -17 * size).all()
 
 
 @pytest.mark.parametrize("H,S,D,causal,o_err,lse_err", [
