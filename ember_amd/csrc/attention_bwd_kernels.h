@@ -232,13 +232,13 @@ __device__ __forceinline__ int dq_turn_expect(const BwdArgs &a, const BwdBlock &
 template <int D>
 constexpr bool kDoneAtOnce = BwdLayout<D>::DB < 4;
 
-// The finished dQ block (rows m0..m0+31) added into dq with atomics;
+// The finished dQ block (rows m0..m0+31) times scale, added into dq with atomics;
 // deterministic mode (kDqOrdered) first waits for its turn (polled: an
 // earlier read of the tile counter) and counts its adds (kDoneAtOnce) or
 // leaves that to the caller.
 template <int D, bool CAUSAL, int DQ>
 __device__ __forceinline__ void dq_store(const BwdArgs &a, const BwdBlock &k, int m0, const f32x16 &qacc,
-                                         int polled)
+                                         float scale, int polled)
 {
     constexpr int DB = BwdLayout<D>::DB;
     const int lane = threadIdx.x & 63;
@@ -256,13 +256,13 @@ __device__ __forceinline__ void dq_store(const BwdArgs &a, const BwdBlock &k, in
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             float *rowp = dqb + (int64_t)(((i >> 2) * 8 + (i & 3)) * k.in_ss);
-            unsafeAtomicAdd(rowp + qoff, qacc[i] * a.scale);
+            unsafeAtomicAdd(rowp + qoff, qacc[i] * scale);
         }
     } else {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             float *rowp = dqb + (int64_t)(((i >> 2) * 8 + (i & 3)) * k.in_ss);
-            if (m0 + acc_row(i, h32) < k.S) unsafeAtomicAdd(rowp + qoff, qacc[i] * a.scale);
+            if (m0 + acc_row(i, h32) < k.S) unsafeAtomicAdd(rowp + qoff, qacc[i] * scale);
         }
     }
     if constexpr (DQ != kDqAtomic && kDoneAtOnce<D>) order_done(k.turns + (m0 >> 4));

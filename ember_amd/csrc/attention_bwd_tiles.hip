@@ -11,7 +11,7 @@
 // the contraction along d they are read as they lie, with the contraction
 // along the rows by the transposing LDS read (ds_read_b64_tr_b16), which hands
 // each lane one column of four rows.  Per block and wave:
-//   S   = Q K^T             beside it: next block's dO split and stored
+//   S   = Q K^T             beside it: this block's dO split and stored
 //   dP  = dO V^T            beside it: P = exp2(S c - lse2), split
 //   dV += P^T dO            beside it: dS = P (dP - delta), split (P and dS
 //                           stand in the accumulators as the operand needs)
@@ -25,7 +25,15 @@
 // have it too; P and dS carry it times the key block's parity, so that dK and
 // dV rows get theirs, and dQ, where the keys' signs cancel, one that
 // alternates from key block to key block.  All come off where a value is
-// scaled anyway.
+// scaled anyway, and 2^32 of scale with them.
+//
+// What the scaled split cannot carry (Q or K from 2^44, V or dO from 2^111,
+// dS from 2^42 on, infinities, NaN) ends a workgroup's walk before that step
+// adds its dQ; the waves then form their dK and dV, and the dQ of the rest of
+// the walk, with the fp32 instruction straight from global memory, at the end
+// of the kernel, where that code takes no registers from the walk.  (Done
+// within the step, S and dP alone, 32 vector operations per step to look for
+// it instead of 16: 4 heads of 300 at D = 128 72.8 us, now 70.4.)
 //
 // What bounds it: at D = 128 one workgroup per CU is one wave per SIMD, so a
 // wave's own waits (four barriers and the LDS reads of each block's first
@@ -89,6 +97,41 @@ __device__ __forceinline__ u32x4 read_columns(const u32x4 *plane, int r0, int r1
     return __builtin_bit_cast(u32x4, Pair{lo, hi});
 }
 
+// P and dP of 32 query rows from m0 and 32 keys from n0 on the fp32 matrix
+// instruction, straight from global memory, for what the split cannot carry;
+// 0 where masked.  Register i holds row acc_row(i, h32), a lane
+// column l32: rows are queries and columns keys, or (KEY_ROWS) the other way.
+template <int D, bool CAUSAL, bool KEY_ROWS>
+__device__ __forceinline__ void block_f32(const BwdArgs &a, int64_t in_base, int64_t out_base, const float *l2p,
+                                          int m0, int n0, f32x16 &p, f32x16 &dp)
+{
+    const int lane = threadIdx.x & 63, h32 = lane >> 5, l32 = lane & 31;
+    const int64_t mr = min(m0 + l32, a.S - 1), nr = min(n0 + l32, a.S - 1);
+    const float *const qr = a.q + in_base + mr * a.in_ss + h32 * (D / 2), *const kr = a.k + in_base + nr * a.in_ss + h32 * (D / 2);
+    const float *const gr = a.dout + out_base + mr * a.out_ss + h32 * (D / 2), *const vr = a.v + in_base + nr * a.in_ss + h32 * (D / 2);
+    f32x16 s = zero16();
+    dp = zero16();
+#pragma unroll 2
+    for (int kk = 0; kk < D / 2; ++kk) {
+        s = KEY_ROWS ? mfma_32x32x2(kr[kk], qr[kk], s) : mfma_32x32x2(qr[kk], kr[kk], s);
+        dp = KEY_ROWS ? mfma_32x32x2(vr[kk], gr[kk], dp) : mfma_32x32x2(gr[kk], vr[kk], dp);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int m = m0 + (KEY_ROWS ? l32 : acc_row(i, h32)), n = n0 + (KEY_ROWS ? acc_row(i, h32) : l32);
+        const bool seen = m < a.S && n < a.S && (!CAUSAL || n <= m);
+        p[i] = seen ? __builtin_amdgcn_exp2f(fmaf(s[i], a.c, -l2p[m])) : 0.0f;
+        dp[i] = seen ? dp[i] : 0.0f;
+    }
+}
+
+__device__ __forceinline__ float not_finite(const f32x16 &v, float probe)
+{
+#pragma unroll
+    for (int i = 0; i < 16; ++i) probe = fmaf(v[i], 0.0f, probe);
+    return probe;
+}
+
 template <int D, bool CAUSAL, int DQ>
 __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(BwdArgs a)
 {
@@ -96,8 +139,8 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     constexpr int U = T::U, KS = T::KS, DB = T::DB, G = T::G;
     __shared__ u32x4 Kp[3 * T::KPL], Qp[3 * T::QPL], Gp[3 * T::QPL];
     __shared__ u32x4 Sp_own[T::kShared ? 1 : 3 * T::SPL];
-    __shared__ unsigned found_in[kWaves];
     __shared__ float St[2][2 * kBq];  // lse2 and delta of a block, two blocks
+    __shared__ int lost_at;  // the step that met what the split cannot carry
     u32x4 *const Sp = T::kShared ? Gp : Sp_own;
 
     const int tid = threadIdx.x;
@@ -121,6 +164,17 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     const unsigned parity = (unsigned)(kb & 1) << 31;
     const unsigned ksgn = sign_of(n0w + l32);   // on this lane's key of K and V, so on S and dP
     const unsigned psgn = ksgn ^ parity;        // on P and dS
+    // Operands are scaled as split_bf16.h says: S, dP, dK, dV and dQ carry
+    // 2^32, P and dS 2^16.  Q and K are multiplied in two steps, so that
+    // elements from 2^44 on become infinite and S NaN: below that no sum in S
+    // passes 2^95 (one of minus infinity would hide in a weight of 0), and dQ,
+    // summed over 128 keys, is finite where dS with its scale is below 2^59.
+    constexpr float kLift = 0x1p84f, kDrop = 0x1p-68f, kUnscale = 1.0f / (kSplitScale * kSplitScale);
+    static_assert(kLift * kDrop == kSplitScale, "in all");
+    // A scale that would become denormal is lost too.
+    const float cs = a.scale > 0.0f && a.scale < 0x1p-94f ? NAN : flip(a.c * kUnscale, ksgn);
+    const float pscale = flip(kSplitScale, psgn);
+    const float dqscale = flip(a.scale * kUnscale, parity);
 
     BwdBlock k;
     k.dqp = a.dq + in_base;
@@ -150,9 +204,12 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
         }
     };
     unsigned part[3][2];
-    // Pair i (of 4) of group g; every second one stores half a unit of each plane.
-    auto split_store = [&](const float (&reg)[G][8], float f, int g, int i, u32x4 *to) {
-        split_pair_full(reg[g][2 * i] * f, reg[g][2 * i + 1] * f, part[0][i & 1], part[1][i & 1], part[2][i & 1]);
+    // Pair i (of 4) of group g of Q or dO; every second one stores half a unit
+    // of each plane.
+    auto split_store = [&](bool q, int g, int i, u32x4 *to) {
+        const float x = q ? qreg[g][2 * i] * kLift * kDrop : greg[g][2 * i] * kSplitScale;
+        const float y = q ? qreg[g][2 * i + 1] * kLift * kDrop : greg[g][2 * i + 1] * kSplitScale;
+        split_pair(x, y, part[0][i & 1], part[1][i & 1], part[2][i & 1]);
         if (i & 1) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
             const int e = ti + kThreads * g;
@@ -173,14 +230,9 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     load_stats(qstart * kBq);
 
     // K of the workgroup's keys to LDS, V of this lane's key to registers
-    // (rows past S re-read row S - 1; their P is 0).  The split of very small
-    // numbers, dS = P (dP - delta) among them, would lose bits
-    // (split_bf16.h), so an input that is below 2^-63 throughout is scaled by
-    // 2^32 as it is split, dS with dO and V, and the results are scaled back,
-    // all of it exact.  For K and V the workgroup's keys decide, for Q and dO
-    // their first block (with a scale from there, rows below 2^95 are right).
+    // (rows past S re-read row S - 1; their P is 0).
     Split8 vf[KS];
-    float kscale, vscale, qscale, gscale;
+    bool klost;  // K cannot be carried: not even a dS of 0 may meet it
     {
         constexpr int N = T::KPL / kThreads;
         f32x4 kr[N][2], vr[KS][2];
@@ -195,47 +247,23 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
         for (int ks = 0; ks < KS; ++ks)
             vr[ks][0] = *(const f32x4 *)(vsrc + 16 * ks), vr[ks][1] = *(const f32x4 *)(vsrc + 16 * ks + 4);
 
-        unsigned kbits = 0, vbits = 0, qbits = 0, gbits = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-#pragma unroll
-            for (int it = 0; it < N; ++it) kbits |= float_bits(kr[it][j / 4][j % 4]);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) vbits |= float_bits(vr[ks][j / 4][j % 4]);
-            if (T::QPL >= kThreads || tid < T::QPL)
-#pragma unroll
-                for (int g = 0; g < G; ++g) qbits |= float_bits(qreg[g][j]), gbits |= float_bits(greg[g][j]);
-        }
-        // 1: some value is at least 2^-63; 2: some value is not zero.
-        auto found = [](unsigned bits) {
-            return (__ballot((bits & 0x60000000u) != 0) != 0 ? 1u : 0u) | (__ballot((bits & 0x7fffffffu) != 0) != 0 ? 2u : 0u);
-        };
-        auto scale_of = [](unsigned f) { return (f & 3) == 2 ? 0x1p32f : 1.0f; };
-        const unsigned mine = found(kbits) | found(qbits) << 2 | found(gbits) << 4 | found(vbits) << 6;
-        if (lane == 0) found_in[w] = mine;
-        __syncthreads();
-        const unsigned all = __builtin_amdgcn_readfirstlane(found_in[0] | found_in[1] | found_in[2] | found_in[3]);
-        kscale = scale_of(all), qscale = scale_of(all >> 2), gscale = scale_of(all >> 4), vscale = scale_of(all >> 6);
-
+        float probe = 0.0f;
 #pragma unroll
         for (int it = 0; it < N; ++it) {
             const int i = it * kThreads + tid, r = i / U, u = i % U;
-            const float f = flip(kscale, sign_of(n0 + r));
+            const float f = flip(kDrop, sign_of(n0 + r));
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = kr[it][j / 4][j % 4] * f;
-            Split8 sp;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                {
-                unsigned h, m, l;
-                split_pair_full(v[2 * j], v[2 * j + 1], h, m, l);
-                sp.part[0][j] = h, sp.part[1][j] = m, sp.part[2][j] = l;
+            for (int j = 0; j < 8; ++j) {
+                v[j] = kr[it][j / 4][j % 4] * kLift * f;
+                probe = fmaf(v[j], 0.0f, probe);
             }
+            const Split8 sp = split8(v);
 #pragma unroll
             for (int pl = 0; pl < 3; ++pl) Kp[pl * T::KPL + T::template unit<U>(r, u)] = sp.part[pl];
         }
-        const float f = flip(vscale, ksgn);
+        klost = __ballot(probe != 0.0f) != 0;
+        const float f = flip(kSplitScale, ksgn);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             float v[8];
@@ -244,11 +272,6 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             vf[ks] = split8(v);
         }
     }
-    // S c = sacc * cs; dP and dS carry gscale * vscale, and so delta does.
-    const float cs = flip(a.c, ksgn) / (qscale * kscale), dscale = gscale * vscale;
-    BwdArgs aq = a;  // what dq_store reads
-    aq.scale = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                             float_bits(flip(a.scale / (dscale * kscale), parity))));
 
     f32x16 dvacc[DB], dkacc[DB];
 #pragma unroll
@@ -295,7 +318,7 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             for (int t = 0; t < 6; ++t) mfma_split_term(t, x[c & 1], y[c & 1], sacc);
 #pragma unroll
             for (int u = 0; u < 4 * G; ++u)
-                if (u * KS / (4 * G) == c) split_store(greg, gscale, u / 4, u % 4, Gp);
+                if (u * KS / (4 * G) == c) split_store(false, u / 4, u % 4, Gp);
             __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();  // dO complete
@@ -317,13 +340,12 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
                 const int r = i + j;
                 p[j] = __builtin_amdgcn_exp2f(fmaf(sacc[r], cs, -l2v[r >> 2][r & 3]));
                 if (MASK) p[j] = mask_t - m0 > 8 * (r >> 2) + (r & 3) ? 0.0f : p[j];
-                p[j] = flip(p[j], psgn);
+                p[j] *= pscale;
                 sacc[r] = p[j];
             }
             unsigned h, m, l;
             split_pair(p[0], p[1], h, m, l);
             Split8 &f = pf[i / 8];
-            asm volatile("" : "+v"(h), "+v"(m), "+v"(l));  // here, not behind the branch below
             f.part[0][i / 2 % 4] = h, f.part[1][i / 2 % 4] = m, f.part[2][i / 2 % 4] = l;
         };
         auto read_g = [&](int c) {
@@ -355,36 +377,15 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             __builtin_amdgcn_sched_barrier(0);
         }
 
-        // What the split cannot carry (split_bf16.h): S and dP again with the
-        // fp32 instruction, straight from global memory, so that an infinite
-        // key that gets no weight stays without.  (dV, dK and dQ of what an
-        // infinity does reach are not finite, and may be NaN.)
-        float probe = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) probe = fmaf(pacc[i], 0.0f, fmaf(sacc[i], 0.0f, probe));
-        if (__ballot(probe != 0.0f) != 0) {
-            const int64_t mr = min(m0 + lq, S - 1), nr = min(key, S - 1);
-            const float *qr = qbase + mr * a.in_ss + lh * (D / 2), *gr = gbase + mr * a.out_ss + lh * (D / 2);
-            const float *kr = a.k + in_base + nr * a.in_ss + lh * (D / 2), *vr = a.v + in_base + nr * a.in_ss + lh * (D / 2);
-            sacc = zero16();
-            pacc = zero16();
-            for (int kk = 0; kk < D / 2; ++kk) {
-                sacc = mfma_32x32x2(qr[kk], kr[kk], sacc);
-                pacc = mfma_32x32x2(gr[kk], vr[kk], pacc);
-            }
-            sacc *= flip(qscale * kscale, ksgn);
-            pacc *= flip(gscale * vscale, ksgn);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) p_pair(2 * u);
-        }
-
         // ---- dV; beside it dS ----
+        float probe = 0.0f;  // not finite if some dS is not, and from about 2^58 on
         auto ds_pair = [&](int i) {
             float d[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int r = i + j;
-                d[j] = sacc[r] * fmaf(pacc[r], flip(1.0f, ksgn), -dlv[r >> 2][r & 3]);
+                d[j] = sacc[r] * fmaf(pacc[r], flip(kUnscale, ksgn), -dlv[r >> 2][r & 3]);
+                probe = fmaf(d[j], 0x1p70f, probe);
             }
             unsigned h, m, l;
             split_pair(d[0], d[1], h, m, l);
@@ -442,8 +443,10 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
                 if (g * 2 * DB / 4 == c) ds_store(g);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (tid < 2 * kBq) St[(qb + 1 - qstart) & 1][tid] = tid < kBq ? streg : streg * dscale;
+        if (tid < 2 * kBq) St[(qb + 1 - qstart) & 1][tid] = streg;
+        if ((klost || __ballot(!(fabsf(probe) < INFINITY)) != 0) && lane == 0) lost_at = qb;
         __syncthreads();  // dS complete, every wave done with Q
+        const int lost = lost_at;
 
         // ---- dQ over this wave's share of the keys; beside it the next
         // block's Q is split and stored ----
@@ -459,19 +462,22 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             for (int t = 0; t < 6; ++t) mfma_split_term(t, x[c & 1], y[c & 1], qacc);
 #pragma unroll
             for (int u = 0; u < 4 * G; ++u)
-                if (u * NC / (4 * G) == c) split_store(qreg, qscale, u / 4, u % 4, Qp);
+                if (u * NC / (4 * G) == c) split_store(true, u / 4, u % 4, Qp);
             __builtin_amdgcn_sched_barrier(0);
         }
         load_rows(qbase, a.in_ss, m_of(qb + 2), qreg);
         load_stats(m_of(qb + 2));
-        dq_store<D, CAUSAL, Q>(aq, k, m0, qacc, polled);
+        if (__builtin_amdgcn_readfirstlane(lost) >= 0) return false;
+        dq_store<D, CAUSAL, Q>(a, k, m0, qacc, dqscale, polled);
         if (Q != kDqAtomic && !kDoneAtOnce<D>) order_done(k.turns + (m0 >> 4));
         __syncthreads();  // the next Q complete, every wave done with dS
+        return true;
     };
 
 #pragma unroll
-    for (int u = 0; u < 4 * G; ++u) split_store(qreg, qscale, u / 4, u % 4, Qp);
-    if (tid < 2 * kBq) St[0][tid] = tid < kBq ? streg : streg * dscale;
+    for (int u = 0; u < 4 * G; ++u) split_store(true, u / 4, u % 4, Qp);
+    if (tid < 2 * kBq) St[0][tid] = streg;
+    if (tid == 0) lost_at = -1;
     load_rows(qbase, a.in_ss, m_of(qstart + 1), qreg);
     load_stats(m_of(qstart + 1));
     __syncthreads();
@@ -482,9 +488,11 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
         // a second one made the compiler spill.)
         const int masked = D == 32 ? k.nq : n0w + kBkw > S ? k.nq : CAUSAL ? min(k.nq, qstart + kBk / kBq) : qstart;
         int qb = qstart;
-        for (; qb < masked; ++qb) step(std::true_type{}, mode, qb);
+        for (; qb < masked; ++qb)
+            if (!step(std::true_type{}, mode, qb)) return;
         if constexpr (D > 32)
-            for (; qb < k.nq; ++qb) step(std::false_type{}, mode, qb);
+            for (; qb < k.nq; ++qb)
+                if (!step(std::false_type{}, mode, qb)) return;
     };
     if constexpr (DQ == kDqAtomic) {
         walk(std::integral_constant<int, kDqAtomic>{});
@@ -501,19 +509,68 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             walk(std::integral_constant<int, kDqOrdered>{});
     }
 
+    // What the split cannot carry: the walk ended before dQ of the step
+    // lost_at was added, or dK or dV is not finite.  The wave's dK and dV with
+    // the fp32 instruction, and below dQ's rest.
+    const int lost = __builtin_amdgcn_readfirstlane(lost_at);
+    float probe = 0.0f, dkscale = a.scale * kUnscale, dvscale = kUnscale;
+    unsigned signs = 0x80000000u;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) probe = not_finite(dkacc[db], not_finite(dvacc[db], probe));
+    if (__ballot(probe != 0.0f) != 0 || lost >= 0) {
+        dkscale = a.scale, dvscale = 1.0f, signs = 0;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) dvacc[db] = zero16(), dkacc[db] = zero16();
+        for (int m0 = qstart * kBq; m0 < S; m0 += kBq) {
+            f32x16 p, dp;
+            block_f32<D, CAUSAL, false>(a, in_base, out_base, l2p, m0, n0w, p, dp);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int m = m0 + acc_row(i, h32);  // below S_pad
+                const int64_t mr = min(m, S - 1);
+                const float ds = p[i] * (dp[i] - dlp[m]);
+                const float *const gr = gbase + mr * a.out_ss + l32, *const qr = qbase + mr * a.in_ss + l32;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    dvacc[db] = mfma_32x32x2(p[i], gr[32 * db], dvacc[db]);
+                    dkacc[db] = mfma_32x32x2(ds, qr[32 * db], dkacc[db]);
+                }
+            }
+        }
+    }
+
     // dK (scaled) and dV rows of this wave's keys: register i -> key
     // n0w + acc_row(i, h32), lane -> d = 32 db + l32.
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int n = n0w + acc_row(i, h32);
         if (n >= S) continue;
-        const unsigned sg = sign_of(n) ^ parity;
+        const unsigned sg = (sign_of(n) ^ parity) & signs;
         const int64_t off = in_base + (int64_t)n * a.in_ss + l32;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-            a.dk[off + 32 * db] = fmaf(dkacc[db][i], flip(a.scale / (dscale * qscale), sg), 0.0f);
-            a.dv[off + 32 * db] = fmaf(dvacc[db][i], flip(1.0f / gscale, sg), 0.0f);
+            a.dk[off + 32 * db] = fmaf(dkacc[db][i], flip(dkscale, sg), 0.0f);
+            a.dv[off + 32 * db] = fmaf(dvacc[db][i], flip(dvscale, sg), 0.0f);
         }
+    }
+    if (lost < 0) return;
+    const int dblk = w % DB, nb = n0 + (w / DB) * T::NK;
+    for (int m0 = lost * kBq; m0 < S; m0 += kBq) {
+        int polled = 0;
+        if (DQ != kDqAtomic) polled = order_poll(k.turns + (m0 >> 4));
+        const float delta = dlp[m0 + l32];
+        f32x16 qacc = zero16();
+        for (int n = nb; n < nb + T::NK; n += 32) {
+            f32x16 p, dp;
+            block_f32<D, CAUSAL, true>(a, in_base, out_base, l2p, m0, n, p, dp);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int64_t nr = min(n + acc_row(i, h32), S - 1);
+                qacc = mfma_32x32x2(p[i] * (dp[i] - delta), a.k[in_base + nr * a.in_ss + 32 * dblk + l32], qacc);
+            }
+        }
+        dq_store<D, CAUSAL, DQ>(a, k, m0, qacc, a.scale, polled);
+        if (DQ != kDqAtomic && !kDoneAtOnce<D>) order_done(k.turns + (m0 >> 4));
     }
 }
 

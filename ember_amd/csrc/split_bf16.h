@@ -52,19 +52,6 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kSplitScale = 0x1p16f;
 
-// A row whose largest magnitude is below 2^-95 (and not 0) is left to the
-// fp32 instruction, so that a row that stays keeps lo down to 2^-39 of its
-// largest element.  Kernels collect the bits of a row's elements with OR (one
-// operation per pair): the exponent fields' top three bits then tell.
-__device__ __forceinline__ bool split_tiny(unsigned bits)
-{
-    return (bits & 0x7fffffffu) != 0 && (bits & 0x70000000u) == 0;
-}
-__device__ __forceinline__ unsigned float_bits(float x)
-{
-    return __builtin_bit_cast(unsigned, x);
-}
-
 // The sign bit of row or column i: the top bit of i times 2^32 / golden ratio,
 // which alternates evenly over every stride of i.
 __device__ __forceinline__ unsigned sign_of(int i)
@@ -87,20 +74,6 @@ __device__ __forceinline__ unsigned pack_bf16(float x0, float x1)
 __device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &m, unsigned &l)
 {
     h = pack_bf16(x0, x1);
-    x0 -= __builtin_bit_cast(float, h << 16);
-    x1 -= __builtin_bit_cast(float, h & 0xffff0000u);
-    m = pack_bf16(x0, x1);
-    x0 -= __builtin_bit_cast(float, m << 16);
-    x1 -= __builtin_bit_cast(float, m & 0xffff0000u);
-    l = pack_bf16(x0, x1);
-}
-
-// The same for values up to the largest fp32 number, which bf16 would round up
-// to infinity.
-__device__ __forceinline__ void split_pair_full(float x0, float x1, unsigned &h, unsigned &m, unsigned &l)
-{
-    const float top = __builtin_bit_cast(float, 0x7f7f0000u);
-    h = pack_bf16(__builtin_amdgcn_fmed3f(x0, -top, top), __builtin_amdgcn_fmed3f(x1, -top, top));
     x0 -= __builtin_bit_cast(float, h << 16);
     x1 -= __builtin_bit_cast(float, h & 0xffff0000u);
     m = pack_bf16(x0, x1);

@@ -1,7 +1,7 @@
 """The split-bf16 backward (attn_bwd_kernel) where it can go wrong: lengths
 around its key and query blocks, the rule that chooses it at D = 64, values
-that the split cannot carry, and its error against float64 next to the fp32
-instruction's."""
+that the split cannot carry, operands of every magnitude, and its error
+against float64 next to the fp32 instruction's."""
 
 import numpy as np
 import pytest
@@ -12,11 +12,11 @@ from ember_amd import capi
 pytestmark = pytest.mark.gpu
 
 
-def _ref(q, k, v, do, causal):
+def _ref(q, k, v, do, causal, scale=None):
     """float64 O, LSE, dQ, dK, dV of (S, D) operands."""
     q, k, v, do = (x.astype(np.float64) for x in (q, k, v, do))
     S, D = q.shape
-    scale = np.float64(np.float32(1 / np.sqrt(D)))
+    scale = np.float64(np.float32(1 / np.sqrt(D) if scale is None else scale))
     s = q @ k.T * scale
     if causal:
         s[np.triu(np.ones((S, S), bool), 1)] = -np.inf
@@ -34,17 +34,17 @@ def _data(H, S, D, seed):
     return [rng.standard_normal((1, H, S, D), dtype=np.float32) for _ in range(4)]
 
 
-def _backward(q, k, v, do, causal, heads):
+def _backward(q, k, v, do, causal, heads, scale=None):
     """The kernel's gradients, with O and LSE from the reference at `heads`
     (zero elsewhere: nothing is read across heads), the references and the log."""
     o, lse = np.zeros_like(q), np.zeros(q.shape[:3], np.float32)
     refs = []
     for h in heads:
-        r = _ref(q[0, h], k[0, h], v[0, h], do[0, h], causal)
+        r = _ref(q[0, h], k[0, h], v[0, h], do[0, h], causal, scale)
         o[0, h], lse[0, h] = r[0], r[1]
         refs.append(r[2:])
     log = []
-    got = G.attention_bwd(q, k, v, o, lse, do, causal, log=log)
+    got = G.attention_bwd(q, k, v, o, lse, do, causal, scale, log=log)
     return got, refs, log
 
 
@@ -142,6 +142,96 @@ def test_zero_first_rows_and_large_values(H, S, D, causal):
         np.testing.assert_allclose(got[2][0, h] / big, rv / float(big), rtol=1e-3, atol=2e-4)
         np.testing.assert_allclose(got[0][0, h], rq, rtol=1e-3, atol=2e-4)
         np.testing.assert_allclose(got[1][0, h], rk, rtol=1e-3, atol=2e-4)
+
+
+def _check_sizes(got, refs, heads, rel=1e-5):
+    """Each gradient to `rel` of its largest element (denormal: to 2^-148)."""
+    for h, ref in zip(heads, refs):
+        for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+            assert np.abs(g[0, h] - r).max() <= rel * np.abs(r).max() + 2.0 ** -148, f"{name} head {h}"
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("eq,ek,es", [(-122, 122, 0), (122, -122, 0), (-120, 40, 80), (30, -120, 90), (-60, -60, 120),
+                                      (60, 40, -100), (20, 20, -40)])
+def test_scores_of_small_and_large_operands(H, S, D, causal, eq, ek, es):
+    """Q and K of 2^eq and 2^ek, denormal ones too, which the scale 2^es
+    brings back to ordinary scores."""
+    q, k, v, do = _data(H, S, D, 6)
+    heads = (0, H - 1)
+    q, k, scale = np.ldexp(q, eq), np.ldexp(k, ek), np.ldexp(1 / np.sqrt(D), es)
+    got, refs, _ = _backward(q, k, v, do, causal, heads, scale)
+    _check_sizes(got, refs, heads)
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("exponent", [-112, -118, -124])
+def test_small_gradients_beside_large_ones(H, S, D, causal, exponent):
+    """dO rows of 2^exponent among ordinary ones and after a block of zeros:
+    their dQ, and dK where the ordinary rows' Q is 0, keep their precision."""
+    q, k, v, do = _data(H, S, D, 7)
+    large = np.arange(S) % 7 == 3
+    do[:, :, :32] = 0
+    do[:, :, ~large] *= np.float32(2.0 ** exponent)
+    q[:, :, large] = 0
+    heads = (0, H - 1)
+    got, refs, _ = _backward(q, k, v, do, causal, heads)
+    for h, (rq, rk, rv) in zip(heads, refs):
+        # 2^-149 per product: dS itself may be denormal.
+        assert (np.abs(got[0][0, h] - rq)[~large] <= 1e-5 * np.abs(rq[~large]).max() + S * 2.0 ** -149).all()
+        assert (np.abs(got[1][0, h] - rk) <= 1e-5 * np.abs(rk).max() + S * 2.0 ** -149).all()
+        np.testing.assert_allclose(got[2][0, h], rv, rtol=1e-3, atol=2e-4)
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+def test_tiny_weights_of_large_gradients(H, S, D, causal):
+    """Weights of exp(-86), 2^-124, times dO of 2^60 (dV)."""
+    q, k, v, do = _data(H, S, D, 8)
+    q[:], k[:] = 0, 0
+    q[..., 0] = np.sqrt(D)
+    k[:, :, 1:, 0] = np.random.default_rng(9).uniform(-86.4, -85, (1, H, S - 1))
+    do *= np.float32(2.0 ** 60)
+    heads = (0, H - 1)
+    got, refs, _ = _backward(q, k, v, do, causal, heads)
+    for h, (_, _, rv) in zip(heads, refs):
+        p = np.exp(k[0, h, 1:, 0].astype(np.float64))
+        size = np.cumsum(np.abs(do[0, h, ::-1]), 0)[::-1][1:] if causal else np.abs(do[0, h]).sum(0)[None]
+        # The exponent, about 124 in base 2, has an ulp of 2^-17: 2^-18 ln 2
+        # each in the product with the scale and in the difference from lse.
+        assert (np.abs(got[2][0, h][1:] - rv[1:]) <= 2.0 ** -17 * p[:, None] * size).all()
+
+
+@pytest.mark.parametrize("H,S,D,causal", FORMS)
+@pytest.mark.parametrize("which,exponent", [("q", 50), ("k", 50), ("v", 113), ("do", 113), ("ds", 0)])
+def test_large_rows_go_on_with_the_fp32_instruction(H, S, D, causal, which, exponent):
+    """One row that the scaled split cannot carry, in the middle of the walk:
+    the workgroups that meet it end theirs in fp32, with the same gradients
+    on every run in deterministic order."""
+    q, k, v, do = _data(H, S, D, 10)
+    row, f = S // 2 + 5, np.float32(2.0 ** exponent)
+    heads = (0, H - 1)
+    if which == "ds":                                  # dS of about 2^52, dQ' of 2^60
+        v *= np.float32(2.0 ** 26)
+        do[:, :, row] *= np.float32(2.0 ** 26)
+    elif which in ("q", "k"):
+        x, y = (q, k) if which == "q" else (k, q)
+        x[:, :, row, 3], y[..., 3] = f, 0              # finds nothing to multiply but 0
+    else:
+        x, y = (v, do) if which == "v" else (do, v)
+        x[:, :, row, 3] = f
+        y[..., 3] /= f
+    ref = None
+    for det in (False, True, True):
+        capi.set_deterministic(det)
+        try:
+            got, refs, _ = _backward(q, k, v, do, causal, heads)
+        finally:
+            capi.set_deterministic(False)
+        _check_sizes(got, refs, heads)
+        if det and ref is not None:
+            assert all(np.array_equal(a, b) for a, b in zip(got, ref))
+        ref = got if det else None
+    assert capi.deterministic_timeouts() == 0
 
 
 @pytest.mark.parametrize("H,S,D,causal,errs", [
