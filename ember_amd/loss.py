@@ -30,11 +30,14 @@ class MSELoss(Loss):
 
     Equal shapes take one fused pass (``_mse_loss``) that returns the same
     float sum as ``sum(diff * diff)`` and the gradient ``(2/n) * diff`` bit
-    for bit; broadcasting shapes compose the operators as the reference."""
+    for bit; broadcasting shapes compose the operators as the reference.  That
+    gradient is handed out once, and a further ``backward`` forms another:
+    callers may write into what they get."""
 
     def __init__(self) -> None:
         self.diff: Tensor | None = None
         self.grad: Tensor | None = None
+        self.pair: tuple | None = None
         self.n = 0
 
     def forward(self, pred: Tensor, target: Tensor) -> float:
@@ -42,16 +45,20 @@ class MSELoss(Loss):
         if isinstance(pred, Tensor) and isinstance(target, Tensor) and pred.shape == target.shape:
             total, g = C._mse_loss(pred._core, target._core, 2.0 / self.n if self.n else 0.0)
             self.diff, self.grad = None, Tensor._from_core(g, pred.shape)
+            self.pair = tuple(Tensor._from_core(x._core, x.shape) for x in (pred, target))
             return total / self.n
-        self.grad = None
+        self.grad = self.pair = None
         self.diff = pred - target
         return _sum(self.diff * self.diff) / self.n
 
     def backward(self) -> Tensor:
         if self.grad is not None:
-            return self.grad
+            grad, self.grad = self.grad, None
+            return grad
         if self.diff is None:
-            raise RuntimeError("forward() must run before backward()")
+            if self.pair is None:
+                raise RuntimeError("forward() must run before backward()")
+            self.diff = self.pair[0] - self.pair[1]
         return (2.0 / self.n) * self.diff
 
 
@@ -62,8 +69,8 @@ class CrossEntropyLoss(Loss):
     shift; backward (softmax(pred) - target) / batch.
 
     Equal shapes take one fused pass (``_cross_entropy_loss``) that forms the
-    gradient with the probabilities; broadcasting shapes compose the operators
-    as the reference."""
+    gradient with the probabilities, handed out once as MSELoss's is;
+    broadcasting shapes compose the operators as the reference."""
 
     def __init__(self) -> None:
         self.probs: Tensor | None = None
@@ -89,7 +96,8 @@ class CrossEntropyLoss(Loss):
         if self.probs is None or self.target is None:
             raise RuntimeError("forward() must run before backward()")
         if self.grad is not None:
-            return self.grad
+            grad, self.grad = self.grad, None
+            return grad
         return (self.probs - self.target) / self.n
 
 

@@ -116,3 +116,21 @@ def test_most_rows():
             got = np.empty(part, np.float32)
             L.copy_from_device(got.ctypes.data, a.ptr + 4 * first, got.nbytes)
             assert (got == want).all()
+
+
+@pytest.mark.parametrize("cls", [loss.CrossEntropyLoss, loss.MSELoss])
+def test_each_backward_gives_a_gradient_of_its_own(cls):
+    """What a caller does to the tensor it got, in place or through its
+    buffer, does not reach the next call's."""
+    x, t = _case(7, 50, 11)
+    fn = cls()
+    fn(Tensor(x), Tensor(t))
+    first = fn.backward()
+    want = first.to_np()
+    first *= 3.0
+    second = fn.backward()
+    np.testing.assert_array_equal(second.to_np(), want)
+    L = capi.lib()
+    assert L.hipMemset(C.c_void_p(second._core.data_ptr), 0, C.c_size_t(4 * x.size)) == 0
+    assert not second.to_np().any()
+    np.testing.assert_array_equal(fn.backward().to_np(), want)
