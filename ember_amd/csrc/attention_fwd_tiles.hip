@@ -125,8 +125,8 @@ __device__ __forceinline__ void rows_f32(const FwdArgs &a, int b, int hh, int bh
 
 // Query blocks of a workgroup (see launch_waves for which launch takes which):
 //   kOne   one block of 32 NW queries, causally the long walks first;
-//   kBoth  (causal) blocks nqb - 1 - p and p of 16 NW queries, half the waves
-//          each: the second block's key tiles are the first ones of the first
+//   kBoth  (causal, NW = 8) blocks nqb - 1 - p and p of 128 queries, half the
+//          waves each: the second block's key tiles are the first ones of the first
 //          block's, staged once for both;
 //   kTurn  (causal, NW = 8) blocks nqb - 1 - p and p of 256 queries one after
 //          the other: the same number of key tiles for every workgroup.
@@ -454,19 +454,14 @@ int launch_waves(const FwdArgs &args)
     const double cus = ncu > 0 ? ncu : 256;
     const int nqb4 = (args.S + 127) / 128, nqb8 = (args.S + 255) / 256;
     if constexpr (CAUSAL) {
-        // Both blocks of a pair at once where the pairs fit one round.
-        // Measured (us: both / 4 waves, one block / 8 waves, one block):
-        // 32 heads of 1024 at D = 128 101 / 105 / 127, 64 heads 111 / 128 /
-        // 133, 32 of 2048 at D = 64 110 / 128 / 148, 40 of 640 41 / 39 / 50.
+        // Both blocks of a pair at once where the pairs fit one round; beyond,
+        // single blocks (65 heads of 1024 at D = 64: 76 us, 92 as pairs of
+        // 64-query blocks in workgroups of four waves).  Measured (us: both /
+        // 4 waves, one block / 8 waves, one block): 32 heads of 1024 at D =
+        // 128 101 / 105 / 127, 64 heads 111 / 128 / 133, 32 of 2048 at D = 64
+        // 110 / 128 / 148, 40 of 640 41 / 39 / 50.
         const double pairs = (double)((nqb4 + 1) / 2) * args.nbh;
         if (nqb4 >= 4 && pairs <= cus) return launch<D, CAUSAL, 8, kBoth>(args, nqb4);
-        // A sixteenth over: pairs of 64-query blocks, four waves, three
-        // workgroups per CU.  65 heads of 1024 at D = 64: 91 us (the fp32
-        // instruction's kernel 151); single blocks take 78, but the mask
-        // tests of the paired launch stand on this shape.
-        const int nqb2 = (args.S + 63) / 64;
-        if (D < 128 && nqb4 >= 4 && pairs <= cus + cus / 16)
-            return launch<D, CAUSAL, 4, kBoth>(args, nqb2);
     }
     // Workgroups of 4 waves while that spreads the queries better: relative
     // times of the busiest CU, in units of an 8-wave workgroup's walk.  One

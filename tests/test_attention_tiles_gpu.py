@@ -43,11 +43,11 @@ def _check(q, k, v, causal, heads, log=None):
 @pytest.mark.parametrize("H,S,D,causal", [
     # 4 waves, one block: one key past a tile, one short of it, one past a block
     (70, 129, 32, False), (70, 191, 32, True), (70, 129, 64, False), (66, 257, 64, False),
-    (70, 159, 128, False), (66, 161, 128, True), (65, 255, 128, False),
+    (70, 159, 128, False), (66, 161, 128, True), (65, 255, 128, False), (65, 960, 64, True),
     # 8 waves, one block
     (300, 129, 128, False), (260, 257, 64, False), (300, 385, 32, True), (130, 511, 128, False),
     # two blocks at once: even and odd counts, a last block of one row
-    (40, 513, 64, True), (64, 641, 128, True), (30, 385, 32, True), (65, 960, 64, True),
+    (40, 513, 64, True), (64, 641, 128, True), (30, 385, 32, True), (64, 960, 64, True),
     # two blocks in turn
     (256, 512, 64, True), (256, 400, 128, True),
 ])

@@ -25,7 +25,7 @@ backward (dQ, dK, dV, with O and LSE passed in unchanged):
     sum (1e-5) instead.
 Two tilings (forward): the same head through a split-key kernel (in a
 small launch) and through attn_fwd_kernel (single or paired query blocks), attn_fwd_head or
-attn_fwd_wave_pair (among 65 heads) agrees within the north-star tolerance and with the CPU oracle, and
+attn_fwd_wave_pair (among 65 heads, 64 for the pairs) agrees within the north-star tolerance and with the CPU oracle, and
 both pass the cutoff check above.  Every launch's first and last head are also held to the oracle
 at the north-star tolerance.
 
@@ -126,6 +126,7 @@ FWD_CASES = [
     ("attn_fwd_kernel", 1, 65, 300, 64),
     ("attn_fwd_kernel", 1, 130, 1024, 128),    # block pairs would exceed one round: single blocks
     ("attn_fwd_kernel", 1, 200, 1024, 64),
+    ("attn_fwd_kernel", 1, 65, 1024, 64),         # one head more than the pairs take
     ("attn_fwd_kernel", 1, 65, 200, 32),
     ("attn_fwd_kernel_pairs", 1, 33, 1024, 128),  # blocks nqb - 1 - p and p per workgroup
     ("attn_fwd_kernel_pairs", 1, 40, 1024, 64),
@@ -189,18 +190,20 @@ def test_two_tilings_same_mask(S, D, H1, alone, other):
     four waves over interleaved 32-key tiles; as head 0 of H1) and through a
     second kernel (128-query blocks over 64-key tiles, whole heads staged in
     LDS with 16-query chunks, or one wave per pair of 32-query blocks) as
-    head 7 of 65: both pass the cutoff check with the same
+    head 7 of 65 (of 64 for paired blocks, the most heads whose pairs run in
+    one round): both pass the cutoff check with the same
     cutoffs for that head, and agree with the oracle and with each other
     within the north-star tolerance."""
     rng = np.random.default_rng(S + D)
     q1, k1, v1 = (_rand((1, H1, S, D), rng) for _ in range(3))
-    qs, ks, vs = (_rand((1, 65, S, D), rng) for _ in range(3))
+    heads = 64 if other == "attn_fwd_kernel_pairs" else 65
+    qs, ks, vs = (_rand((1, heads, S, D), rng) for _ in range(3))
     for big, one in ((qs, q1), (ks, k1), (vs, v1)):
         big[0, 7] = one[0, 0]
     one_rounds = _cutoff_rounds(H1, S, S)
     many_rounds = []
     for r, cut1 in enumerate(one_rounds):
-        cut = _cutoff_rounds(65, S, S + r)[0]
+        cut = _cutoff_rounds(heads, S, S + r)[0]
         cut[7] = cut1[0]
         many_rounds.append(cut)
     G.say(f"two tilings S={S} D={D}: {alone}")
