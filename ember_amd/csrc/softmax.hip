@@ -217,7 +217,8 @@ struct LossArgs {
 };
 
 // a / n with r = 1 / n: the quotient corrected by its exact remainder
-// (Markstein's method), and the special cases of a division.
+// (Markstein's method), and the special cases of a division; n within
+// 2^-100 .. 2^100, so that r is an ordinary number.
 __device__ __forceinline__ float divide_by(float a, float n, float r)
 {
     const float q = a * r;
@@ -391,7 +392,8 @@ extern "C" int cross_entropy_loss(const float *logits, const float *target, floa
     char *ws = (char *)scratch(kScratchSum, (size_t)blocks * sizeof(double) + 16);
     if (!ws) return EMBER_ERR_OUT_OF_MEMORY;
     const HostSum result((uint64_t *)(ws + (size_t)blocks * sizeof(double)), true);
-    const LossArgs a = {logits, target, probs, grad, (double *)ws, result.out(), rows, L, n};
+    const bool ordinary = fabsf(n) >= 0x1p-100f && fabsf(n) <= 0x1p100f;  // divide_by
+    const LossArgs a = {logits, target, probs, grad, (double *)ws, result.out(), rows, L, ordinary ? n : 1.0f};
     if (L <= 16) launch_loss<16, 1, 1>(a, blocks);
     else if (L <= 32) launch_loss<32, 1, 1>(a, blocks);
     else if (by_block) hipLaunchKernelGGL(cross_entropy_long, dim3(blocks), dim3(256), 0, 0, a);
@@ -408,5 +410,9 @@ extern "C" int cross_entropy_loss(const float *logits, const float *target, floa
         else if (L <= 512) launch_loss<64, 8, 1>(a, blocks);
         else launch_loss<64, 16, 1>(a, blocks);
     }
-    return launch_ok("cross_entropy_loss") ? result.read(total, "cross_entropy_loss") : EMBER_ERR_DEVICE;
+    if (!launch_ok("cross_entropy_loss")) return EMBER_ERR_DEVICE;
+    const int64_t size = (int64_t)rows * L, part = int64_t(1) << 30;
+    for (int64_t i = 0; !ordinary && i < size; i += part)
+        truediv_scalar(grad + i, n, grad + i, (int)std::min(part, size - i));
+    return result.read(total, "cross_entropy_loss");
 }

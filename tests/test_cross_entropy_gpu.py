@@ -134,3 +134,22 @@ def test_each_backward_gives_a_gradient_of_its_own(cls):
     assert L.hipMemset(C.c_void_p(second._core.data_ptr), 0, C.c_size_t(4 * x.size)) == 0
     assert not second.to_np().any()
     np.testing.assert_array_equal(fn.backward().to_np(), want)
+
+
+@pytest.mark.parametrize("n", [1e-40, 1e-38, -2.0, 0.25, 3e38, 0.0, np.inf, np.nan])
+def test_any_divisor(n):
+    """The C entry's n: (probs - target) / n as fp32 divides, also where 1 / n
+    is denormal or infinite."""
+    rows, classes = 9, 100
+    x, t = _case(rows, classes, 12)
+    t[:] = 0
+    t[:, 3] = 1
+    L, total = capi.lib(), C.c_float()
+    dx, dt = DeviceArray.from_numpy(x), DeviceArray.from_numpy(t)
+    p, g = DeviceArray(x.shape), DeviceArray(x.shape)
+    capi.check(L.cross_entropy_loss(dx.ptr, dt.ptr, p.ptr, g.ptr, rows, classes, n, C.byref(total)), "cross_entropy_loss")
+    with np.errstate(all="ignore"):
+        want = (p.numpy() - t) / np.float32(n)
+    # Equal but for the sign of a zero.
+    np.testing.assert_array_equal(g.numpy() + np.float32(0), want + np.float32(0))
+    assert total.value == pytest.approx(_ref(x, t, 1)[0], rel=2e-6)
