@@ -29,7 +29,6 @@ struct GemmArgs {
     float *c;
     int n, m, k;
     int lda, ldb;        // row pitch of a and b as stored (k or n; m or k)
-    int ta, tb;          // a stored k x n / b stored m x k
     int64_t sa, sb, sc;  // batch strides (elements)
     int tiles_n, tiles_m;
     int tile0;           // first tile of this launch
@@ -518,8 +517,6 @@ int gemm_launch(const float *a, const float *b, float *out, int batch, int n, in
     g.n = n;
     g.m = m;
     g.k = k;
-    g.ta = ta;
-    g.tb = tb;
     g.lda = ta ? n : k;
     g.ldb = tb ? k : m;
     g.sa = (int64_t)n * k;

@@ -1,8 +1,9 @@
 // mfma.h -- fp32 matrix-core helpers for gfx950 (CDNA4).
 //
-// All tiles in this library are built from v_mfma_f32_32x32x2f32: one wave
-// (64 lanes) multiplies a 32x2 A slice by a 2x32 B slice into a 32x32 fp32
-// accumulator held as 16 floats per lane.  Operand and result placement
+// v_mfma_f32_32x32x2f32: one wave (64 lanes) multiplies a 32x2 A slice by a
+// 2x32 B slice into a 32x32 fp32 accumulator held as 16 floats per lane.  (The
+// larger products run on the bf16 instruction of the same accumulator layout,
+// split_bf16.h.)  Operand and result placement
 // (checked on the device with an in-bounds probe):
 //   A[m][k]  : lane l supplies m = l % 32, k = l / 32
 //   B[k][n]  : lane l supplies n = l % 32, k = l / 32

@@ -146,9 +146,11 @@ float sum(const float *a, int size);
  * sum and mul_scalar.  Synchronises (the loss is read back). */
 int mse_loss(const float *pred, const float *target, float *grad, int size, float scale, float *loss);
 /* Ember's CrossEntropyLoss over (rows, classes) in one pass
- * (ember/loss/losses.py:29-56): probs = softmax(logits), grad = (probs -
- * target) / n, *total = sum of target * log_softmax(logits), in the fp32
- * operations of the composed operators but for the order of a row's sum.  No
+ * (ember/loss/losses.py:29-56).  Per row, in fp32: m = max, e = exp(logits -
+ * m), s = sum of e in a tree, probs = e * (1 / s), grad = (probs - target) /
+ * n; *total = sum of target * (logits - m - log(s)), added in double.  (The
+ * composed operators sum s in index order and form probs as exp of the
+ * rounded log-probability, which is a few roundings further off.)  No
  * reference counterpart as one symbol.  Synchronises (the sum is read back). */
 int cross_entropy_loss(const float *logits, const float *target, float *probs, float *grad, int rows, int classes,
                        float n, float *total);
