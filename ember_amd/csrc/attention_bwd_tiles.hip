@@ -38,13 +38,13 @@
 // What bounds it: at D = 128 one workgroup per CU is one wave per SIMD, so a
 // wave's own waits (four barriers and the LDS reads of each block's first
 // operands) leave the matrix cores idle: B4 H32 S4096 D128 causal busy 52 % of
-// cycles at 1.93 GHz (power limit), LDS busy 35 %, a third of that in bank
-// conflicts of the transposing reads.  Hence the vector work laid beside the
+// cycles at 1.86 GHz (power limit), with 4.8 vector instructions to a matrix
+// one, and bank conflicts of the transposing reads in 12 %.  Hence the vector work laid beside the
 // products, and operands read a chunk ahead.  Against the kernel on the fp32
-// instruction that it replaced: B4 H32 S4096 D128 causal 10711 -> 8112 us
-// (128 -> 169 TFLOP/s), 30 heads of 777 at D = 128 264 -> 170, 32 heads of 1024
-// causal 335 -> 211, 4 heads of 300 110 -> 70; D = 32, 64 heads of 1000 causal
-// 164 -> 148; in deterministic order 11028 -> 8281 at the first.  Error against
+// instruction that it replaced: B4 H32 S4096 D128 causal 10740 -> 8090 us
+// (128 -> 170 TFLOP/s; in deterministic order 4 % longer), 30 heads of 777 at
+// D = 128 265 -> 172, 32 heads of 1024 causal 336 -> 212, 4 heads of 300 109 ->
+// 70; D = 32, 64 heads of 1000 causal 166 -> 154.  Error against
 // float64 (relative 2-norm, the first, dQ, dK, dV): 6.0e-7, 1.6e-6, 1.6e-6 ->
 // 5.2e-7, 1.2e-6, 1.2e-6.
 #include "attention_bwd_kernels.h"

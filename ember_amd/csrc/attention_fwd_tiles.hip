@@ -20,14 +20,15 @@
 // the S products of tile t.
 //
 // What bounds it: the power limit, through the matrix cores and the vector
-// work beside them (B4 H32 S4096 D128 causal: cores busy 57 % of cycles at
-// 1.90 GHz, vector instructions 29 %; without a limit the clock is 2.4 GHz).
+// work beside them (B4 H32 S4096 D128 causal: cores busy 66 % of cycles at
+// 1.74 GHz, 4.3 vector instructions to a matrix one; without a limit the clock
+// is 2.4 GHz).
 // Tried against it and dropped: the two waves of a SIMD half a tile apart, so
 // that one's softmax meets the other's products (a third V buffer; 2971
 // against 2821 us there).  Against the fp32 instruction's kernel it replaced:
-// B4 H32 S4096 D128 causal 4050 -> 2782 us (136 -> 198 TFLOP/s), B8 H16 S2048
-// D64 causal 539 -> 386 (127 -> 178), B2 H8 S4096 D128 956 -> 610 (144 -> 225),
-// 30 heads of 777 at D = 128 111 -> 85; error of O against float64 5.7e-7 ->
+// B4 H32 S4096 D128 causal 3980 -> 2660 us (138 -> 207 TFLOP/s), B8 H16 S2048
+// D64 causal 539 -> 388 (127 -> 177), B2 H8 S4096 D128 963 -> 624 (143 -> 220),
+// 30 heads of 777 at D = 128 111 -> 86; error of O against float64 5.7e-7 ->
 // 4.6e-7, 4.1e-7 -> 3.3e-7, 1.3e-6 -> 1.0e-6, 6.7e-7 -> 5.4e-7.
 #include <math.h>
 

@@ -177,9 +177,9 @@ struct Operand {
 
 // A TM x TN block of out per workgroup of WR x WC waves, each 32*RB x 32*CB.
 // What bounds it: the matrix cores, and at 4096^3 the power limit with them
-// (72 % of cycles busy, at 1.70 GHz; the same launch on constant operands
-// holds 2.28 GHz): 933 -> 601 us, 147 -> 228 TFLOP/s against the fp32
-// instruction's kernel this replaced.  Splitting costs 6.5 vector operations
+// (78 % of cycles busy, at 1.64 GHz; the same launch on constant operands
+// holds 2.28 GHz): 933 -> 584 us, 147 -> 235 TFLOP/s against the fp32
+// instruction's kernel this replaced (573 to 627 us over cards).  Splitting costs 6.5 vector operations
 // per element staged (2.6 per matrix instruction in the 256 x 256 tile, 4 are
 // free beside one), so operands are split once, when they enter LDS, and not
 // by each wave that reads them.

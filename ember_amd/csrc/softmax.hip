@@ -187,7 +187,7 @@ void launch_wave(const float *a, float *out, int rows, int L)
 // a workgroup each and three passes, of which the second and third hit the
 // caches.
 // Measured, value and gradient with the sum read back, composed and here: 8192
-// x 1000 179 and 46 us (the kernel 40 us without the next row's loads and with
+// x 1000 179 and 45 us (the kernel 40 us without the next row's loads and with
 // a second expf and a division per element, 30 with them: 4.4 TB/s).
 constexpr int kLossBlocks = 1024;  // 4 workgroups of 4 waves per CU
 
