@@ -27,8 +27,8 @@
 // alternates from key block to key block.  All come off where a value is
 // scaled anyway, and 2^32 of scale with them.
 //
-// What the scaled split cannot carry (Q or K from 2^44, V or dO from 2^111,
-// dS from 2^42 on, infinities, NaN) ends a workgroup's walk before that step
+// What the scaled split cannot carry (Q or K from 2^44, V or dO from 2^111
+// on, dS so large that dQ might pass 2^96, infinities, NaN) ends a workgroup's walk before that step
 // adds its dQ; the waves then form their dK and dV, and the dQ of the rest of
 // the walk, with the fp32 instruction straight from global memory, at the end
 // of the kernel, where that code takes no registers from the walk.  (Done
@@ -112,9 +112,14 @@ __device__ __forceinline__ void block_f32(const BwdArgs &a, int64_t in_base, int
     f32x16 s = zero16();
     dp = zero16();
 #pragma unroll 2
-    for (int kk = 0; kk < D / 2; ++kk) {
-        s = KEY_ROWS ? mfma_32x32x2(kr[kk], qr[kk], s) : mfma_32x32x2(qr[kk], kr[kk], s);
-        dp = KEY_ROWS ? mfma_32x32x2(vr[kk], gr[kk], dp) : mfma_32x32x2(gr[kk], vr[kk], dp);
+    for (int kk = 0; kk < D / 2; kk += 4) {
+        const f32x4 qv = *(const f32x4 *)(qr + kk), kv = *(const f32x4 *)(kr + kk);
+        const f32x4 gv = *(const f32x4 *)(gr + kk), vv = *(const f32x4 *)(vr + kk);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s = KEY_ROWS ? mfma_32x32x2(kv[j], qv[j], s) : mfma_32x32x2(qv[j], kv[j], s);
+            dp = KEY_ROWS ? mfma_32x32x2(vv[j], gv[j], dp) : mfma_32x32x2(gv[j], vv[j], dp);
+        }
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -141,6 +146,7 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     __shared__ u32x4 Sp_own[T::kShared ? 1 : 3 * T::SPL];
     __shared__ float St[2][2 * kBq];  // lse2 and delta of a block, two blocks
     __shared__ int lost_at;  // the step that met what the split cannot carry
+    __shared__ float kmax_in[kWaves];
     u32x4 *const Sp = T::kShared ? Gp : Sp_own;
 
     const int tid = threadIdx.x;
@@ -167,8 +173,7 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     // Operands are scaled as split_bf16.h says: S, dP, dK, dV and dQ carry
     // 2^32, P and dS 2^16.  Q and K are multiplied in two steps, so that
     // elements from 2^44 on become infinite and S NaN: below that no sum in S
-    // passes 2^95 (one of minus infinity would hide in a weight of 0), and dQ,
-    // summed over 128 keys, is finite where dS with its scale is below 2^59.
+    // passes 2^95 (one of minus infinity would hide in a weight of 0).
     constexpr float kLift = 0x1p84f, kDrop = 0x1p-68f, kUnscale = 1.0f / (kSplitScale * kSplitScale);
     static_assert(kLift * kDrop == kSplitScale, "in all");
     // A scale that would become denormal is lost too.
@@ -232,7 +237,8 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
     // K of the workgroup's keys to LDS, V of this lane's key to registers
     // (rows past S re-read row S - 1; their P is 0).
     Split8 vf[KS];
-    bool klost;  // K cannot be carried: not even a dS of 0 may meet it
+    bool klost;    // K cannot be carried: not even a dS of 0 may meet it
+    float dslimit;  // dS times this overflows before dQ, its sum over 128 keys
     {
         constexpr int N = T::KPL / kThreads;
         f32x4 kr[N][2], vr[KS][2];
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
         for (int ks = 0; ks < KS; ++ks)
             vr[ks][0] = *(const f32x4 *)(vsrc + 16 * ks), vr[ks][1] = *(const f32x4 *)(vsrc + 16 * ks + 4);
 
-        float probe = 0.0f;
+        float probe = 0.0f, kmax = 0.0f;
 #pragma unroll
         for (int it = 0; it < N; ++it) {
             const int i = it * kThreads + tid, r = i / U, u = i % U;
@@ -257,12 +263,20 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
             for (int j = 0; j < 8; ++j) {
                 v[j] = kr[it][j / 4][j % 4] * kLift * f;
                 probe = fmaf(v[j], 0.0f, probe);
+                kmax = fmaxf(kmax, fabsf(v[j]));
             }
             const Split8 sp = split8(v);
 #pragma unroll
             for (int pl = 0; pl < 3; ++pl) Kp[pl * T::KPL + T::template unit<U>(r, u)] = sp.part[pl];
         }
         klost = __ballot(probe != 0.0f) != 0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) kmax = fmaxf(kmax, __shfl_xor(kmax, o));
+        if (lane == 0) kmax_in[w] = kmax;
+        __syncthreads();
+        kmax = fmaxf(fmaxf(kmax_in[0], kmax_in[1]), fmaxf(kmax_in[2], kmax_in[3]));
+        // The sum over dS below may cancel once: a factor 2 beside the 2^7.
+        dslimit = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(float_bits(kmax * 0x1p9f)));
         const float f = flip(kSplitScale, ksgn);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -378,14 +392,14 @@ __global__ __launch_bounds__(kThreads, D == 32 ? 2 : 1) void attn_bwd_kernel(Bwd
         }
 
         // ---- dV; beside it dS ----
-        float probe = 0.0f;  // not finite if some dS is not, and from about 2^58 on
+        float probe = 0.0f;  // not finite if some dS is not or dQ might not be
         auto ds_pair = [&](int i) {
             float d[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int r = i + j;
                 d[j] = sacc[r] * fmaf(pacc[r], flip(kUnscale, ksgn), -dlv[r >> 2][r & 3]);
-                probe = fmaf(d[j], 0x1p70f, probe);
+                probe = fmaf(d[j], dslimit, probe);
             }
             unsigned h, m, l;
             split_pair(d[0], d[1], h, m, l);

@@ -58,6 +58,10 @@ __device__ __forceinline__ unsigned sign_of(int i)
 {
     return ((unsigned)i * 0x9E3779B9u) & 0x80000000u;
 }
+__device__ __forceinline__ unsigned float_bits(float x)
+{
+    return __builtin_bit_cast(unsigned, x);
+}
 __device__ __forceinline__ float flip(float x, unsigned sign)
 {
     return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) ^ sign);
