@@ -112,8 +112,8 @@ def test_infinite_keys_get_no_weight(H, S, D, causal):
 @pytest.mark.parametrize("which", ["q", "k", "v", "do"])
 @pytest.mark.parametrize("exponent", [-100, -115])
 def test_tiny_inputs_keep_their_precision(H, S, D, causal, which, exponent):
-    """One input below what three bf16 parts can hold: gradients to fp32
-    precision relative to their size."""
+    """One input below what three bf16 parts can hold without a scale:
+    gradients to fp32 precision relative to their size."""
     f = np.float32(2.0 ** exponent)
     data = dict(zip(("q", "k", "v", "do"), _data(H, S, D, 3)))
     data[which] *= f
@@ -128,8 +128,8 @@ def test_tiny_inputs_keep_their_precision(H, S, D, causal, which, exponent):
 
 @pytest.mark.parametrize("H,S,D,causal", FORMS)
 def test_zero_first_rows_and_large_values(H, S, D, causal):
-    """A first query block of zeros, then rows whose dO is about 2^100:
-    the first rows' scale holds for them."""
+    """A first query block of zeros, then rows whose dO is about 2^100: dV
+    passes what its scaled sum can hold and is formed again in fp32."""
     q, k, v, do = _data(H, S, D, 5)
     do[0, :, :32] = 0
     q[0, :, :32] = 0

@@ -92,8 +92,8 @@ def test_infinite_values(H, S, D, causal):
 @pytest.mark.parametrize("H,S,D,causal", FORMS)
 @pytest.mark.parametrize("exponent", [-100, -120])
 def test_tiny_values_keep_their_precision(H, S, D, causal, exponent):
-    """V below what three bf16 parts can hold: O to fp32 precision relative
-    to V's size."""
+    """V below what three bf16 parts can hold without a scale: O to fp32
+    precision relative to V's size."""
     q, k, v = _qkv(H, S, D, 3)
     v *= np.float32(2.0 ** exponent)
     o, _ = G.attention_fwd(q, k, v, causal)

@@ -92,8 +92,8 @@ def test_magnitudes_next_to_the_largest_float():
 @pytest.mark.parametrize("exponent", [-99, -101, -110, -125])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
 def test_tiny_rows_keep_their_precision(exponent, ta, tb):
-    """Rows of a and columns of b below what three bf16 parts can hold; the
-    other operand brings the results back into range."""
+    """Rows of a and columns of b below what three bf16 parts can hold without
+    a scale; the other operand brings the results back into range."""
     n, k, m = 90, 200, 75
     a, b = _u((n, k), 7), _u((k, m), 8) * np.float32(2.0 ** 60)
     a[10:20] *= np.float32(2.0 ** exponent)
