@@ -1,8 +1,8 @@
 """The split-bf16 GEMM where it can go wrong: tile edges and short last k-slabs
 of each tile shape and orientation, operands that do not start on 16 bytes,
 values the split cannot carry (infinities, NaN, magnitudes next to the largest
-float), elements of every magnitude beside larger ones, and its error against float64 next to the fp32
-chain's."""
+float), elements of every magnitude beside larger ones, extents up to 2^31 - 1,
+and its error against float64 next to the fp32 chain's."""
 
 import ctypes as C
 
